@@ -353,10 +353,12 @@ static int ensure_layer_exact(pqa_ctx* ctx, int layer, const char* fn) {
     const int n = p.n_embd, rows = (int)ctx->kv_dim;
     const size_t fk = pqa::exact_matrix_floats(p.wtype[1], rows, n);
     const size_t fv = pqa::exact_matrix_floats(p.wtype[2], rows, n);
+    if (int rc = ensure_batch(ctx, (size_t)rows * n, fn)) return rc;
     float* buf = nullptr;
     if (int rc = hip_check(ctx, hipMalloc(&buf, (fk + fv) * 4), fn)) return rc;
-    hipError_t e = pqa::prepare_exact_matrix(p.wtype[1], p.w[1], p.stride[1], rows, n, buf, ctx->stream);
-    if (e == hipSuccess) e = pqa::prepare_exact_matrix(p.wtype[2], p.w[2], p.stride[2], rows, n, buf + fk, ctx->stream);
+    hipError_t e = pqa::prepare_exact_matrix(p.wtype[1], p.w[1], p.stride[1], rows, n, ctx->wf32, buf, ctx->stream);
+    if (e == hipSuccess)
+        e = pqa::prepare_exact_matrix(p.wtype[2], p.w[2], p.stride[2], rows, n, ctx->wf32, buf + fk, ctx->stream);
     if (int rc = hip_check(ctx, e, fn)) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipFree(buf);
@@ -366,18 +368,32 @@ static int ensure_layer_exact(pqa_ctx* ctx, int layer, const char* fn) {
     return PQA_OK;
 }
 
+// Whether attn_k / attn_v read the inputs' image in the Q8_0 order or the chain
+// order (a layer may mix them), and the floats one image of n_tok inputs takes.
+static size_t image_floats(const pqa_proj_weights& p, int n_tok) {
+    const bool qk = p.wtype[1] == pqa::GG_Q8_0, qv = p.wtype[2] == pqa::GG_Q8_0;
+    return std::max(pqa::ordered_image_floats(qk, n_tok, p.n_embd), pqa::ordered_image_floats(qv, n_tok, p.n_embd));
+}
+
 // k[t * ldo + r] and v[t * ldo + r] = the attn_k / attn_v matmul_bias of token
-// t in the reference's order (pqa_exact.hip), bit-exact.
-static int exact_kv(pqa_ctx* ctx, int layer, int n_tok, const float* xb, float* k, float* v, int ldo, const char* fn) {
+// t in the reference's order (pqa_exact.hip), bit-exact. image: image_floats of
+// workspace.
+static int exact_kv(pqa_ctx* ctx, int layer, int n_tok, const float* xb, float* image, float* k, float* v, int ldo,
+                    const char* fn) {
     if (int rc = ensure_layer_exact(ctx, layer, fn)) return rc;
     const auto& p = ctx->proj[layer];
     const int n = p.n_embd, rows = (int)ctx->kv_dim;
     const float* wk = p.exact;
     const float* wv = p.exact + pqa::exact_matrix_floats(p.wtype[1], rows, n);
-    hipError_t e = pqa::launch_ordered_project(p.wtype[1], wk, rows, n, xb, n, n_tok, p.b[1], p.btype[1], k, ldo,
-                                               ctx->stream);
+    const pqa::OrderedProj kv[2] = {{p.wtype[1], wk, p.b[1], p.btype[1], k}, {p.wtype[2], wv, p.b[2], p.btype[2], v}};
+    const bool qk = p.wtype[1] == pqa::GG_Q8_0, qv = p.wtype[2] == pqa::GG_Q8_0;
+    hipError_t e = pqa::launch_ordered_image(qk, xb, n, n_tok, n, image, ctx->stream);
     if (e == hipSuccess)
-        e = pqa::launch_ordered_project(p.wtype[2], wv, rows, n, xb, n, n_tok, p.b[2], p.btype[2], v, ldo, ctx->stream);
+        e = pqa::launch_ordered_project(kv, qk == qv ? 2 : 1, rows, n, image, n_tok, ldo, ctx->stream);
+    if (e == hipSuccess && qk != qv) {
+        e = pqa::launch_ordered_image(qv, xb, n, n_tok, n, image, ctx->stream);
+        if (e == hipSuccess) e = pqa::launch_ordered_project(kv + 1, 1, rows, n, image, n_tok, ldo, ctx->stream);
+    }
     return hip_check(ctx, e, fn);
 }
 
@@ -399,19 +415,22 @@ struct SplitBufs {
     _Float16* x3;
     float* x_inv;
     float* y;
+    float* image;  // of X, for the reference-order projection (image_floats, 0: none)
 };
 
-static size_t split_need(int n_tok, int n, size_t total) {
-    return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2) + up256((size_t)n_tok * 4) + (size_t)n_tok * total * 4;
+static size_t split_need(int n_tok, int n, size_t total, size_t image) {
+    return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2) + up256((size_t)n_tok * 4) + up256((size_t)n_tok * total * 4) +
+           image * 4;
 }
 
-static int ensure_split(pqa_ctx* ctx, int n_tok, int n, size_t total, SplitBufs* sb, const char* fn) {
+static int ensure_split(pqa_ctx* ctx, int n_tok, int n, size_t total, size_t image, SplitBufs* sb, const char* fn) {
     const size_t xb = up256((size_t)n_tok * 2 * pqa::k_half(n) * 2), xs = up256((size_t)n_tok * 4);
-    if (int rc = grow_split(ctx, split_need(n_tok, n, total), fn)) return rc;
+    if (int rc = grow_split(ctx, split_need(n_tok, n, total, image), fn)) return rc;
     char* base = (char*)ctx->bsplit;
     sb->x3 = (_Float16*)base;
     sb->x_inv = (float*)(base + xb);
     sb->y = (float*)(base + xb + xs);
+    sb->image = (float*)(base + xb + xs + up256((size_t)n_tok * total * 4));
     return PQA_OK;
 }
 
@@ -428,7 +447,7 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
     const int kh = pqa::k_half(n);
     const _Float16* w3 = (const _Float16*)p.split;
     *w_inv = (const float*)((const char*)p.split + up256(total * 2 * kh * 2));
-    if (int rc = ensure_split(ctx, n_tok, n, total, sb, fn)) return rc;
+    if (int rc = ensure_split(ctx, n_tok, n, total, q_only ? image_floats(p, n_tok) : 0, sb, fn)) return rc;
     pqa::launch_split2(xb, n_tok, n, sb->x3, kh, sb->x_inv, ctx->stream);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
     // Y[n_tok][total] = X_hi W_hi^T + X_hi W_lo^T + X_lo W_hi^T (the q rows come first)
@@ -480,7 +499,7 @@ extern "C" int pqa_qkv_project_batch(pqa_ctx* ctx, int layer, int n_tok, const f
     hipLaunchKernelGGL(pqa::unscale_scatter_kernel, dim3(gx, n_tok), dim3(256), 0, ctx->stream, (const float*)sb.y,
                        (int)total, ncols, w_inv, (const float*)sb.x_inv, sa);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
-    return exact ? exact_kv(ctx, layer, n_tok, xb, k, v, (int)ctx->kv_dim, fn) : PQA_OK;
+    return exact ? exact_kv(ctx, layer, n_tok, xb, sb.image, k, v, (int)ctx->kv_dim, fn) : PQA_OK;
 }
 
 // The prompt path from the normed inputs: the GEMM result goes to the prefill
@@ -503,7 +522,7 @@ extern "C" int pqa_prefill_x(pqa_ctx* ctx, int layer, int start_pos, int n_tok, 
     const auto& p = ctx->proj[layer];
     const int ld = (int)(ctx->q_dim + 2 * ctx->kv_dim);
     if (exact)  // the k and v columns of the GEMM result, in the reference's order
-        if (int rc = exact_kv(ctx, layer, n_tok, xb, sb.y + ctx->q_dim, sb.y + ctx->q_dim + ctx->kv_dim, ld, fn))
+        if (int rc = exact_kv(ctx, layer, n_tok, xb, sb.image, sb.y + ctx->q_dim, sb.y + ctx->q_dim + ctx->kv_dim, ld, fn))
             return rc;
     pqa::PrefillScaled ys;
     ys.y = sb.y;
@@ -528,7 +547,7 @@ static int out_project_batch(pqa_ctx* ctx, int layer, int n_tok, const float* at
     const int n = (int)ctx->q_dim, rows = p.out_rows;
     const int kh = pqa::k_half(n);
     SplitBufs sb;
-    if (int rc = ensure_split(ctx, n_tok, n, (size_t)rows, &sb, fn)) return rc;
+    if (int rc = ensure_split(ctx, n_tok, n, (size_t)rows, 0, &sb, fn)) return rc;
     pqa::launch_split2(attn, n_tok, n, sb.x3, kh, sb.x_inv, ctx->stream);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
     const _Float16* w3 = (const _Float16*)p.out_split;
@@ -577,7 +596,9 @@ extern "C" int pqa_prefill_block(pqa_ctx* ctx, int layer, int start_pos, int n_t
     // every buffer of both GEMMs exists before the first kernel is queued
     const auto& p = ctx->proj[layer];
     const size_t total = ctx->q_dim + 2 * ctx->kv_dim;
-    const size_t need = std::max(split_need(n_tok, p.n_embd, total), split_need(n_tok, (int)ctx->q_dim, p.out_rows));
+    const size_t image = ctx->batch_exact_kv ? image_floats(p, n_tok) : 0;
+    const size_t need =
+        std::max(split_need(n_tok, p.n_embd, total, image), split_need(n_tok, (int)ctx->q_dim, p.out_rows, 0));
     if (int rc = grow_split(ctx, need, fn)) return rc;
     const size_t af = (size_t)n_tok * ctx->q_dim;
     if (af > ctx->battn_floats) {

@@ -12,26 +12,40 @@
 //   Q8_0 rows (:321-340): per 32-element block sum += q * x in order, then
 //   sumf += d * sum in block order;
 //   then out + bias (vec_add).
-// Nothing here reorders a sum: each kernel is a register-tiled VALU GEMM whose
-// lanes each own one chain (or, for Q8_0, whole rows of blocks) of 64 (token,
-// row) pairs and walk that chain's elements in increasing order, with
-// separate multiply and add instructions (built with -ffp-contract=off). MFMA
-// and tree reductions would round differently. The outputs are bit-identical
-// to the reference's matmul_bias built without FMA contraction, like
-// pqa_qkv_project for one token.
+// Nothing here reorders a sum. The vector ALU bounds both halves of it, the
+// products and the ordered additions: it starts a wave's next instruction every
+// 5 cycles but takes one of another wave in between (32 additions: 162 cycles
+// with one wave per SIMD, 80 per wave with two), so waves per SIMD count for
+// twice. The products come from v_mfma_f32_32x32x1_2b with C = 0, 2 x 32 x 32
+// of them round(w * x) in 70 cycles; it shares the vector ALU (no overlap was
+// measured), but takes its operands as one row and one token per lane where a
+// register tile reads 16 values for 64 products. Its bits are v_mul_f32's for
+// subnormals, infinities and NaN alike, up to the sign of a zero (2^27 products
+// of random and special bit patterns compared), which no sum that starts at +0
+// shows. (A shape with K > 1 would fuse its own additions and round otherwise.)
 //
-// ordered_dot_kernel (every type but Q8_0): workgroup = 64 tokens x 64 rows,
-// 8 waves. Wave w owns tokens 8w .. 8w+7; lane = 8 rg + p owns rows
-// 8 rg .. 8 rg+7 and chain c(p) (p < 4: chain p; p >= 4: chain 11 - p, so
-// that chain l+4 sits at lane p ^ 7, DPP row_half_mirror). Per 64-element k
-// tile the operands are staged in LDS with chain c's 8 elements at columns
-// 4c .. 4c+3 (first 32) and 32 + 4c .. +3 (second 32), so a lane reads its
-// chain as two 16-byte words per row. 64 products and 64 sums per lane per
-// element of the chain: the kernel is bound by VALU issue.
+// ordered_kernel: a workgroup of 4 waves owns 32 tokens x 32 rows. The sums of a
+// (token, row) pair run as 8 independent sequences over 64-element stages:
+//   chain types  sequence c = chain c, the stage's elements 8 j + c (j < 8);
+//   Q8_0         sequence c = block c of a round of 8 blocks (4 stages), the
+//                stage's 8 elements j of it.
+// A wave takes two sequences as the MFMA's two blocks (chains q and q + 4, or
+// blocks 2 q and 2 q + 1): 32 sums and 32 products per lane, so that four waves
+// fit a SIMD and a tile alone keeps four busy. No operand is shared between the
+// waves, so LDS would only add instructions, which are what the kernel is short
+// of: both operands come as images in the order the lanes read them (below), two
+// 16-byte loads each per stage, requested two stages ahead (one for Q8_0). At the
+// end (Q8_0: of each round) the waves' sums meet in LDS and each wave finishes a
+// quarter of the tile in the reference's order.
+// K and V together, 2 x 1024 rows x 2560: 2048 tokens 353 us and 9 for the inputs'
+// image (a 64 x 64 register tile with VALU multiplies, a launch each: 506 us); 75
+// tokens 35 + 5 us (226 us). 2048 tokens run at 163 cycles per MFMA and its 32
+// additions, against 152 measured for the two alone.
 //
-// ordered_q8_kernel: workgroup = 64 tokens x 64 rows, 4 waves; thread (tg,
-// rg) owns tokens tg + 16 i and rows rg + 16 j (i, j < 4) over every element
-// in order, one 32-element block per LDS stage.
+// Image of a matrix [rows][n] (n rounded up to whole stages, Q8_0 whole rounds,
+// with zeros): per tile of 32 rows and stage, [wave q][half h][lane][4]: lane l is
+// row l % 32 and the wave's sequence l / 32, the four floats are elements
+// 4 h .. 4 h + 3 of that sequence's 8.
 #include <algorithm>
 
 #include "pqa_device.h"
@@ -39,242 +53,188 @@
 
 namespace pqa {
 
-constexpr int kOrdTile = 64;                      // tokens and rows per workgroup, k elements per stage
-constexpr int kOrdThreads = 512;                  // ordered_dot_kernel
-constexpr int kOrdRowF = kOrdTile + 4;            // LDS row stride in floats (272 bytes: staging writes spread over banks)
-constexpr int kQ8Threads = 256;                   // ordered_q8_kernel
-constexpr int kQ8RowF = 36;                       // LDS row stride of one 32-element block row (+4 floats)
+typedef float floatx32 __attribute__((ext_vector_type(32)));
+
+constexpr int kOrdTile = 32;                      // tokens and rows per workgroup
+constexpr int kOrdK = 64;                         // k elements per stage: 8 of each of the 8 sequences
+constexpr int kOrdThreads = 256;                  // 4 waves
+constexpr int kOrdStageF = kOrdTile * kOrdK;      // floats of one operand's stage
+
+__host__ __device__ inline int ord_stages(bool q8, int n) { return q8 ? (n + 255) / 256 * 4 : (n + kOrdK - 1) / kOrdK; }
+
+// element k of a row: its stage, and its float within the stage's image at lane row `r`
+__device__ __forceinline__ void ord_place(bool q8, int k, int r, int& st, int& f) {
+    int c, j;  // sequence and element of the stage
+    if (q8) {
+        st = (k >> 8) * 4 + ((k >> 3) & 3);
+        c = (k >> 5) & 7;
+        j = k & 7;
+    } else {
+        st = k >> 6;
+        c = k & 7;
+        j = (k >> 3) & 7;
+    }
+    const int q = q8 ? c >> 1 : c & 3, b = q8 ? c & 1 : c >> 2;
+    f = (2 * q + (j >> 2)) * 256 + (32 * b + r) * 4 + (j & 3);
+}
 
 struct OrderedArgs {
-    const float* x;  // [n_tok][ldx] fp32 inputs
-    const float* w;  // [rows][n]: fp32 rows (dequantized), or for Q8_0 the int8 values as floats
-    const float* d;  // Q8_0: [rows][n / 32] block scales; else unused
-    int n_tok, rows, n, ldx;
-    const uint8_t* b;  // bias [rows] (F32 or F16) or null
-    int bt;
-    float* out;  // out[t * ldo + r]
-    int ldo;
+    const float* w[2];  // images of the weight rows (Q8_0: the int8 values as floats)
+    const float* d[2];  // Q8_0: [rows][n / 32] block scales; else unused
+    const uint8_t* b[2];  // bias [rows] (F32 or F16) or null
+    int bt[2];
+    float* out[2];  // out[t * ldo + r]
+    const float* x;  // image of the inputs
+    int n_tok, rows, n, ldo;
+    int rtiles;  // row tiles per matrix
 };
 
 __device__ __forceinline__ float ord_bias(const uint8_t* b, int bt, int r) {
     return bt == GG_F32 ? ((const float*)b)[r] : f16_bits_to_f32(((const uint16_t*)b)[r]);
 }
 
-// 16 bytes of row `row` at element k (k + 4 <= n, or zeros past n; n is a
-// multiple of 4). ALIGNED: the row base is 16-byte aligned.
-template <bool ALIGNED>
-__device__ __forceinline__ float4 ord_load4(const float* base, size_t ld, int row, int k, int n) {
-    if (k >= n) return float4{0.0f, 0.0f, 0.0f, 0.0f};
-    const float* p = base + (size_t)row * ld + k;
-    if constexpr (ALIGNED) return *(const float4*)p;
-    return float4{p[0], p[1], p[2], p[3]};
-}
-
-// chain of lane position p within its 8 lanes (see the file comment)
-__device__ __forceinline__ int ord_chain(int p) { return p < 4 ? p : 11 - p; }
-
-// Natural element k (0..63) of a tile -> LDS column: chain c = k & 7, its
-// element j = k >> 3 at column 32 (j >> 2) + 4 c + (j & 3).
-__device__ __forceinline__ int ord_col(int k) { return 32 * (k >> 5) + 4 * (k & 7) + ((k >> 3) & 3); }
-
-template <bool XALIGNED>
-__global__ __launch_bounds__(kOrdThreads) void ordered_dot_kernel(const OrderedArgs a) {
+template <bool Q8>
+__global__ __launch_bounds__(kOrdThreads, 4) void ordered_kernel(const OrderedArgs a) {
 #pragma clang fp contract(off)
-    __shared__ __attribute__((aligned(16))) float xs[2][kOrdTile * kOrdRowF];
-    __shared__ __attribute__((aligned(16))) float ws[2][kOrdTile * kOrdRowF];
+    constexpr int PD = Q8 ? 2 : 3;  // stages in registers (Q8_0: a third does not fit four waves per SIMD)
+    constexpr int NR = 16;  // results per lane of the whole tile
+    __shared__ float ex[Q8 ? 8 * NR * 64 : 4 * NR * 64];  // [block or wave][result][lane]
+
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int w = tid >> 6;
-    const int p = lane & 7, rg = lane >> 3;
-    const int c = ord_chain(p);
-    const int t0 = blockIdx.y * kOrdTile, r0 = blockIdx.x * kOrdTile;
-    const int ntile = (a.n + kOrdTile - 1) / kOrdTile;
+    const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hb = lane >> 5;
+    const int mat = (int)blockIdx.x >= a.rtiles ? 1 : 0;
+    const int rt = (int)blockIdx.x - mat * a.rtiles;
+    const int r0 = rt * kOrdTile, t0 = (int)blockIdx.y * kOrdTile;
+    const int nst = ord_stages(Q8, a.n);
+    const float* xt = a.x + ((size_t)blockIdx.y * nst * kOrdStageF + 512 * q);
+    const float* wt = a.w[mat] + ((size_t)rt * nst * kOrdStageF + 512 * q);
 
-    // staging: thread tid moves float4 s = tid + 512 i (i < 2) of each
-    // operand tile: tile row s / 16 (clamped to the last token / row), natural
-    // elements 4 (s % 16) .. +3, written to their chain columns
-    int srow[2], sk[2], scol[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int s = tid + kOrdThreads * i;
-        srow[i] = s >> 4;
-        sk[i] = 4 * (s & 15);
-        scol[i] = ord_col(sk[i]);  // elements sk .. sk+3 share chain-element j, chains c .. c+3
-    }
-    auto load = [&](int tile, float4* xr, float4* wr) {
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int k = tile * kOrdTile + sk[i];
-            xr[i] = ord_load4<XALIGNED>(a.x, a.ldx, min(t0 + srow[i], a.n_tok - 1), k, a.n);
-            wr[i] = ord_load4<true>(a.w, a.n, min(r0 + srow[i], a.rows - 1), k, a.n);
-        }
-    };
-    auto store = [&](int buf, const float4* xr, const float4* wr) {
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            float* xd = &xs[buf][srow[i] * kOrdRowF + scol[i]];
-            float* wd = &ws[buf][srow[i] * kOrdRowF + scol[i]];
-            xd[0] = xr[i].x, xd[4] = xr[i].y, xd[8] = xr[i].z, xd[12] = xr[i].w;
-            wd[0] = wr[i].x, wd[4] = wr[i].y, wd[8] = wr[i].z, wd[12] = wr[i].w;
-        }
-    };
-
-    float acc[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) acc[i][j] = 0.0f;
-
-    float4 xr[2], wr[2];
-    load(0, xr, wr);
-    store(0, xr, wr);
-    __syncthreads();
-    for (int tile = 0; tile < ntile; tile++) {
-        const int buf = tile & 1;
-        const bool more = tile + 1 < ntile;
-        if (more) load(tile + 1, xr, wr);
-        const float* xb = &xs[buf][(8 * w) * kOrdRowF + 4 * c];
-        const float* wb = &ws[buf][(8 * rg) * kOrdRowF + 4 * c];
+    floatx4 xv[PD][2], wv[PD][2];
+    auto load = [&](int st, int p) __attribute__((always_inline)) {
+        const size_t o = (size_t)min(st, nst - 1) * kOrdStageF;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            float4 xv[8], wv[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                xv[i] = *(const float4*)(xb + i * kOrdRowF + 32 * h);
-                wv[i] = *(const float4*)(wb + i * kOrdRowF + 32 * h);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const float xe = e == 0 ? xv[i].x : e == 1 ? xv[i].y : e == 2 ? xv[i].z : xv[i].w;
-                        const float we = e == 0 ? wv[j].x : e == 1 ? wv[j].y : e == 2 ? wv[j].z : wv[j].w;
-                        acc[i][j] = acc[i][j] + we * xe;
-                    }
+            xv[p][h] = *(const floatx4*)(xt + o + 256 * h + 4 * lane);
+            wv[p][h] = *(const floatx4*)(wt + o + 256 * h + 4 * lane);
         }
-        if (more) store(buf ^ 1, xr, wr);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx32 acc;  // sums of this wave's two sequences: MFMA result layout, block b at 16 b
+    floatx32 zero;
+#pragma unroll
+    for (int e = 0; e < 32; e++) acc[e] = zero[e] = 0.0f;
+    float sumf[Q8 ? 4 : 1];  // Q8_0: results 4 q .. +3
+#pragma unroll
+    for (int e = 0; e < (Q8 ? 4 : 1); e++) sumf[e] = 0.0f;
+
+    auto compute = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            float x = xv[p][u >> 2][u & 3];
+            asm volatile("" : "+v"(x));  // keeps this MFMA behind the sums before it: one product buffer
+            const floatx32 pr = __builtin_amdgcn_mfma_f32_32x32x1f32(x, wv[p][u >> 2][u & 3], zero, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 32; e++) acc[e] = acc[e] + pr[e];
+            asm volatile("" : "+v"(acc));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+#pragma unroll
+    for (int p = 0; p < PD; p++) load(p, p);
+    auto step = [&](int st, int p) __attribute__((always_inline)) {
+        compute(p);
+        load(st + PD, p);
+                    if constexpr (Q8) {
+                        if ((st & 3) == 3) {
+                            // the round's 8 blocks: d * sum of each, then added in block order
+                            const int blk0 = 2 * (st & ~3), nblk = a.n / 32;
+                            const float* dr = a.d[mat] + (size_t)min(r0 + l32, a.rows - 1) * nblk;
+                            float d[2];
+        #pragma unroll
+                            for (int b = 0; b < 2; b++) d[b] = dr[min(blk0 + 2 * q + b, nblk - 1)];
+                            __syncthreads();  // the last round has been read
+        #pragma unroll
+                            for (int b = 0; b < 2; b++)
+        #pragma unroll
+                                for (int e = 0; e < 16; e++) ex[((2 * q + b) * NR + e) * 64 + lane] = d[b] * acc[16 * b + e];
+                            __syncthreads();
+        #pragma unroll
+                            for (int b = 0; b < 8; b++) {
+                                if (blk0 + b < nblk) {
+        #pragma unroll
+                                    for (int e = 0; e < 4; e++) sumf[e] = sumf[e] + ex[(b * NR + 4 * q + e) * 64 + lane];
+                                }
+                            }
+        #pragma unroll
+                            for (int e = 0; e < 32; e++) acc[e] = 0.0f;
+                        }
+                    }
+    };
+    // whole groups of PD stages, then the rest: without an exit inside the loop
+    // every wait leaves the later stages' loads in flight
+    int st = 0;
+    for (; st + PD <= nst; st += PD) {
+#pragma unroll
+        for (int p = 0; p < PD; p++) step(st + p, p);
+    }
+#pragma unroll
+    for (int p = 0; p < PD - 1; p++)
+        if (st + p < nst) step(st + p, p);
+
+    // chain types: t = chain l + chain l+4, then (t0 + t2) + (t1 + t3)
+    if constexpr (!Q8) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) ex[(q * NR + e) * 64 + lane] = acc[e] + acc[16 + e];
         __syncthreads();
     }
-
-    // t = chain l + chain l+4 (lane p ^ 7), then (t0 + t2) + (t1 + t3): the
-    // partners are symmetric, so all 8 lanes of a group end with the same bits
-    // (a + b == b + a). Lane p then stores token 8w + p's 8 rows.
-    const int tok = t0 + 8 * w + p;
-    float res[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) res[j] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            float v = acc[i][j];
-            v = v + dpp_f<kDppXor7>(v);
-            v = v + dpp_f<kDppXor2>(v);
-            v = v + dpp_f<kDppXor1>(v);
-            if (i == p) res[j] = v;
+    for (int u = 0; u < 4; u++) {
+        const int e = 4 * q + u;  // result register of the MFMA layout
+        float res;
+        if constexpr (Q8) {
+            res = sumf[u];
+        } else {
+            const float* p = ex + e * 64 + lane;
+            res = (p[0] + p[2 * NR * 64]) + (p[NR * 64] + p[3 * NR * 64]);
         }
-    if (tok < a.n_tok) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int r = r0 + 8 * rg + j;
-            if (r < a.rows) a.out[(size_t)tok * a.ldo + r] = a.b ? res[j] + ord_bias(a.b, a.bt, r) : res[j];
+        const int tok = t0 + 8 * q + 4 * hb + u;
+        const int r = r0 + l32;
+        if (tok < a.n_tok && r < a.rows) {
+            const uint8_t* bias = a.b[mat];
+            a.out[mat][(size_t)tok * a.ldo + r] = bias ? res + ord_bias(bias, a.bt[mat], r) : res;
         }
     }
 }
 
-template <bool XALIGNED>
-__global__ __launch_bounds__(kQ8Threads) void ordered_q8_kernel(const OrderedArgs a) {
-#pragma clang fp contract(off)
-    __shared__ __attribute__((aligned(16))) float xs[2][kOrdTile * kQ8RowF];
-    __shared__ __attribute__((aligned(16))) float ws[2][kOrdTile * kQ8RowF];
-    __shared__ float ds[2][kOrdTile];
+// Image of src [rows][ld] (n columns used; any 4-byte alignment), a workgroup per
+// tile and four stages (Q8_0: a round). Rows past the last repeat it, columns
+// past n are zero.
+template <bool Q8>
+__global__ __launch_bounds__(kOrdThreads) void ordered_image_kernel(const float* __restrict__ src, int ld, int rows,
+                                                                    int n, float* __restrict__ dst) {
+    __shared__ __attribute__((aligned(16))) float img[4 * kOrdStageF];
     const int tid = threadIdx.x;
-    const int tg = tid >> 4, rg = tid & 15;
-    const int t0 = blockIdx.y * kOrdTile, r0 = blockIdx.x * kOrdTile;
-    const int nblk = a.n / 32;
-
-    // staging: 64 rows x 8 float4 per operand; thread tid moves float4 s = tid
-    // + 256 i (i < 2): row s / 8, elements 4 (s % 8) .. +3 of the block
-    auto load = [&](int blk, float4* xr, float4* wr, float& dr) {
+    const int nst = ord_stages(Q8, n), st0 = 4 * (int)blockIdx.x, ns = min(4, nst - st0);
+    // thread = column: the tile's rows one after the other, 1 KB of a row at a time
+    const int k = kOrdK * st0 + tid;
+    float v[kOrdTile];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int s = tid + kQ8Threads * i;
-            const int k = 32 * blk + 4 * (s & 7);
-            xr[i] = ord_load4<XALIGNED>(a.x, a.ldx, min(t0 + (s >> 3), a.n_tok - 1), k, a.n);
-            wr[i] = ord_load4<true>(a.w, a.n, min(r0 + (s >> 3), a.rows - 1), k, a.n);
-        }
-        dr = tid < kOrdTile ? a.d[(size_t)min(r0 + tid, a.rows - 1) * nblk + blk] : 0.0f;
-    };
-    auto store = [&](int buf, const float4* xr, const float4* wr, float dr) {
+    for (int r = 0; r < kOrdTile; r++) {
+        const int row = min((int)blockIdx.y * kOrdTile + r, rows - 1);
+        v[r] = k < n ? src[(size_t)row * ld + k] : 0.0f;
+    }
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int s = tid + kQ8Threads * i;
-            *(float4*)&xs[buf][(s >> 3) * kQ8RowF + 4 * (s & 7)] = xr[i];
-            *(float4*)&ws[buf][(s >> 3) * kQ8RowF + 4 * (s & 7)] = wr[i];
-        }
-        if (tid < kOrdTile) ds[buf][tid] = dr;
-    };
-
-    float sumf[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) sumf[i][j] = 0.0f;
-
-    float4 xr[2], wr[2];
-    float dr;
-    load(0, xr, wr, dr);
-    store(0, xr, wr, dr);
+    for (int r = 0; r < kOrdTile; r++) {
+        int st, f;
+        ord_place(Q8, k, r, st, f);
+        img[(st - st0) * kOrdStageF + f] = v[r];
+    }
     __syncthreads();
-    for (int blk = 0; blk < nblk; blk++) {
-        const int buf = blk & 1;
-        const bool more = blk + 1 < nblk;
-        if (more) load(blk + 1, xr, wr, dr);
-        float sum[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) sum[i][j] = 0.0f;
-#pragma unroll 2
-        for (int k4 = 0; k4 < 8; k4++) {
-            float4 xv[4], wv[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                xv[i] = *(const float4*)&xs[buf][(tg + 16 * i) * kQ8RowF + 4 * k4];
-                wv[i] = *(const float4*)&ws[buf][(rg + 16 * i) * kQ8RowF + 4 * k4];
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float xe = e == 0 ? xv[i].x : e == 1 ? xv[i].y : e == 2 ? xv[i].z : xv[i].w;
-                        const float qe = e == 0 ? wv[j].x : e == 1 ? wv[j].y : e == 2 ? wv[j].z : wv[j].w;
-                        sum[i][j] = sum[i][j] + qe * xe;
-                    }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float dj = ds[buf][rg + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; i++) sumf[i][j] = sumf[i][j] + dj * sum[i][j];
-        }
-        if (more) store(buf ^ 1, xr, wr, dr);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int tok = t0 + tg + 16 * i;
-        if (tok >= a.n_tok) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int r = r0 + rg + 16 * j;
-            if (r < a.rows) a.out[(size_t)tok * a.ldo + r] = a.b ? sumf[i][j] + ord_bias(a.b, a.bt, r) : sumf[i][j];
-        }
-    }
+    floatx4* o = (floatx4*)(dst + ((size_t)blockIdx.y * nst + st0) * kOrdStageF);
+    for (int i = tid; i < ns * kOrdStageF / 4; i += kOrdThreads) o[i] = ((const floatx4*)img)[i];
 }
 
 // Q8_0 rows -> the int8 values as floats [rows][n] and the block scales
@@ -291,50 +251,63 @@ __global__ __launch_bounds__(256) void q8_unpack_kernel(const uint8_t* __restric
     for (int j = 0; j < 32; j++) o[j] = (float)(int8_t)b[2 + j];
 }
 
-// Floats of a matrix's prepared copy: [rows][n] (+ [rows][n / 32] for Q8_0).
+// Floats of the image of [rows][n], and of a matrix's prepared copy (Q8_0: the
+// image, then the block scales).
+size_t ordered_image_floats(bool q8, int rows, int n) {
+    return (size_t)((rows + kOrdTile - 1) / kOrdTile) * ord_stages(q8, n) * kOrdStageF;
+}
 size_t exact_matrix_floats(int type, int rows, int n) {
-    return (size_t)rows * n + (type == GG_Q8_0 ? (size_t)rows * (n / 32) : 0);
+    const bool q8 = type == GG_Q8_0;
+    return ordered_image_floats(q8, rows, n) + (q8 ? (size_t)rows * (n / 32) : 0);
 }
 
-hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, int n, float* dst, hipStream_t s) {
-    if (type == GG_Q8_0) {
+hipError_t launch_ordered_image(bool q8, const float* src, int ld, int rows, int n, float* dst, hipStream_t s) {
+    if (rows <= 0 || n <= 0 || ld < n) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((ord_stages(q8, n) + 3) / 4), (unsigned)((rows + kOrdTile - 1) / kOrdTile));
+    if (q8) hipLaunchKernelGGL(ordered_image_kernel<true>, grid, dim3(kOrdThreads), 0, s, src, ld, rows, n, dst);
+    else hipLaunchKernelGGL(ordered_image_kernel<false>, grid, dim3(kOrdThreads), 0, s, src, ld, rows, n, dst);
+    return hipGetLastError();
+}
+
+hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, int n, float* rows_f32, float* dst,
+                                hipStream_t s) {
+    const bool q8 = type == GG_Q8_0;
+    hipError_t e;
+    if (q8) {
         const long long items = (long long)rows * (n / 32);
         hipLaunchKernelGGL(q8_unpack_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s,
-                           (const uint8_t*)w, stride, rows, n, dst, dst + (size_t)rows * n);
-        return hipGetLastError();
+                           (const uint8_t*)w, stride, rows, n, rows_f32, dst + ordered_image_floats(q8, rows, n));
+        e = hipGetLastError();
+    } else {
+        e = launch_dequant_rows(type, w, stride, rows, n, rows_f32, s);
     }
-    return launch_dequant_rows(type, w, stride, rows, n, dst, s);
+    return e != hipSuccess ? e : launch_ordered_image(q8, rows_f32, n, rows, n, dst, s);
 }
 
-hipError_t launch_ordered_project(int type, const float* prepared, int rows, int n, const float* x, int ldx, int n_tok,
-                                  const void* bias, int btype, float* out, int ldo, hipStream_t s) {
-    if (rows <= 0 || n_tok <= 0 || n <= 0 || n % 8 || ldx < n) return hipErrorInvalidValue;
+hipError_t launch_ordered_project(const OrderedProj* p, int nmat, int rows, int n, const float* x_image, int n_tok,
+                                  int ldo, hipStream_t s) {
+    if (rows <= 0 || n_tok <= 0 || n <= 0 || n % 8 || nmat < 1 || nmat > 2) return hipErrorInvalidValue;
+    const bool q8 = p[0].type == GG_Q8_0;
+    if (q8 && n % 32) return hipErrorInvalidValue;
     OrderedArgs a;
-    a.x = x;
-    a.w = prepared;
-    a.d = type == GG_Q8_0 ? prepared + (size_t)rows * n : nullptr;
+    for (int i = 0; i < 2; i++) {
+        const OrderedProj& m = p[i < nmat ? i : 0];
+        if ((m.type == GG_Q8_0) != q8) return hipErrorInvalidValue;
+        a.w[i] = m.prepared;
+        a.d[i] = q8 ? m.prepared + ordered_image_floats(q8, rows, n) : nullptr;
+        a.b[i] = (const uint8_t*)m.bias;
+        a.bt[i] = m.btype;
+        a.out[i] = m.out;
+    }
+    a.x = x_image;
     a.n_tok = n_tok;
     a.rows = rows;
     a.n = n;
-    a.ldx = ldx;
-    a.b = (const uint8_t*)bias;
-    a.bt = btype;
-    a.out = out;
     a.ldo = ldo;
-    const dim3 grid((unsigned)((rows + kOrdTile - 1) / kOrdTile), (unsigned)((n_tok + kOrdTile - 1) / kOrdTile));
-    const bool xal = ((uintptr_t)x & 15) == 0 && ldx % 4 == 0;
-    if (type == GG_Q8_0) {
-        if (n % 32) return hipErrorInvalidValue;
-        if (xal)
-            hipLaunchKernelGGL(ordered_q8_kernel<true>, grid, dim3(kQ8Threads), 0, s, a);
-        else
-            hipLaunchKernelGGL(ordered_q8_kernel<false>, grid, dim3(kQ8Threads), 0, s, a);
-    } else {
-        if (xal)
-            hipLaunchKernelGGL(ordered_dot_kernel<true>, grid, dim3(kOrdThreads), 0, s, a);
-        else
-            hipLaunchKernelGGL(ordered_dot_kernel<false>, grid, dim3(kOrdThreads), 0, s, a);
-    }
+    a.rtiles = (rows + kOrdTile - 1) / kOrdTile;
+    const dim3 grid((unsigned)(a.rtiles * nmat), (unsigned)((n_tok + kOrdTile - 1) / kOrdTile));
+    if (q8) hipLaunchKernelGGL(ordered_kernel<true>, grid, dim3(kOrdThreads), 0, s, a);
+    else hipLaunchKernelGGL(ordered_kernel<false>, grid, dim3(kOrdThreads), 0, s, a);
     return hipGetLastError();
 }
 

@@ -30,9 +30,9 @@ struct pqa_proj_weights {
     // the same for the attn_output rows (pqa_out_project_batch)
     void* out_split = nullptr;
     // the batched path's attn_k and attn_v rows for the reference-order
-    // projection (pqa_exact.hip): fp32 [kv_dim][n_embd] each (Q8_0: the int8
-    // values as floats, then the block scales); made on the first call that
-    // needs them, dropped with the weights
+    // projection (pqa_exact.hip): the image of the fp32 rows each (Q8_0: of the
+    // int8 values as floats, then the block scales); made on the first call
+    // that needs them, dropped with the weights
     float* exact = nullptr;
 };
 
@@ -191,14 +191,27 @@ hipError_t launch_qkv_project(pqa_ctx* ctx, int layer, const float* xb, float* q
 // GGUF rows [rows][n] -> fp32 [rows][n] by the dequantize_row_* expressions
 // (pqa_batch.hip).
 hipError_t launch_dequant_rows(int type, const void* w, int stride, int rows, int n, float* dst, hipStream_t s);
-// The reference-order projection of a prompt (pqa_exact.hip):
-// exact_matrix_floats / prepare_exact_matrix make a matrix's prepared copy
-// from its GGUF rows; launch_ordered_project writes out[t * ldo + r] =
-// matmul_bias of token t's input x[t * ldx ..] for rows r < rows, bit-exact.
+// The reference-order projection of a prompt (pqa_exact.hip).
+// prepare_exact_matrix makes a matrix's prepared copy (exact_matrix_floats of
+// them) from its GGUF rows through rows_f32 ([rows][n] floats of scratch);
+// launch_ordered_image makes the inputs' image (ordered_image_floats), which
+// depends on whether the weights are Q8_0; launch_ordered_project writes, for
+// nmat (1 or 2) matrices of one shape and one kind of image, p.out[t * ldo + r] =
+// matmul_bias of token t's input for rows r < rows, bit-exact.
+struct OrderedProj {
+    int type;
+    const float* prepared;
+    const void* bias;
+    int btype;
+    float* out;
+};
+size_t ordered_image_floats(bool q8, int rows, int n);
 size_t exact_matrix_floats(int type, int rows, int n);
-hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, int n, float* dst, hipStream_t s);
-hipError_t launch_ordered_project(int type, const float* prepared, int rows, int n, const float* x, int ldx, int n_tok,
-                                  const void* bias, int btype, float* out, int ldo, hipStream_t s);
+hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, int n, float* rows_f32, float* dst,
+                                hipStream_t s);
+hipError_t launch_ordered_image(bool q8, const float* src, int ld, int rows, int n, float* dst, hipStream_t s);
+hipError_t launch_ordered_project(const OrderedProj* p, int nmat, int rows, int n, const float* x_image, int n_tok,
+                                  int ldo, hipStream_t s);
 hipError_t launch_out_project(pqa_ctx* ctx, int layer, const float* attn, float* x);
 
 }  // namespace pqa
