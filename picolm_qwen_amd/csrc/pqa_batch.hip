@@ -218,10 +218,12 @@ __global__ __launch_bounds__(256) void unscale_scatter_kernel(const float* __res
 }
 
 // The output projection of a prompt: Y [n_tok][rows] holds attn W_o^T scaled
-// by 2^(s_w + s_x); x[t][r] = x[t][r] + (Y[t][r] * 2^-(s_w + s_x) + b[r]),
-// the reference's matmul_bias then vec_add (cpp/model.hpp:595-600). Thread: 4
-// consecutive rows of one token (rows a multiple of 4).
-__global__ __launch_bounds__(256) void unscale_residual_kernel(const float* __restrict__ Y, int rows,
+// by 2^(s_w + s_x), as the sum of `slices` parts (the GEMM's K ranges); x[t][r] =
+// x[t][r] + (Y[t][r] * 2^-(s_w + s_x) + b[r]), the reference's matmul_bias then
+// vec_add (cpp/model.hpp:595-600). Thread: 4 consecutive rows of one token (rows
+// a multiple of 4).
+__global__ __launch_bounds__(256) void unscale_residual_kernel(const float* __restrict__ Y, int slices,
+                                                               size_t slice_stride, int rows,
                                                                const float* __restrict__ w_inv,
                                                                const float* __restrict__ x_inv,
                                                                const uint8_t* __restrict__ b, int btype,
@@ -229,9 +231,15 @@ __global__ __launch_bounds__(256) void unscale_residual_kernel(const float* __re
     const int t = blockIdx.y;
     const int r = 4 * (blockIdx.x * 256 + threadIdx.x);
     if (r >= rows) return;
-    const floatx4 y = *(const floatx4*)(Y + (size_t)t * rows + r);
+    floatx4 y = *(const floatx4*)(Y + (size_t)t * rows + r);
     const floatx4 wi = *(const floatx4*)(w_inv + r);
     const float xi = x_inv[t];
+#pragma unroll 4
+    for (int s = 1; s < slices; s++) {
+        const floatx4 v = *(const floatx4*)(Y + s * slice_stride + (size_t)t * rows + r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = y[e] + v[e];
+    }
     floatx4* xp = (floatx4*)(x + (size_t)t * rows + r);
     floatx4 o = *xp;
 #pragma unroll
@@ -241,6 +249,24 @@ __global__ __launch_bounds__(256) void unscale_residual_kernel(const float* __re
         o[e] = o[e] + v;
     }
     *xp = o;
+}
+
+// y[t][c] = the sum of the GEMM's K slices part[s][t][c] in slice order, c < cols
+// (an even number) of y's ld columns. Thread: 2 columns of one token.
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int slices,
+                                                         size_t slice_stride, int cols, float* __restrict__ y, int ld) {
+    const int t = blockIdx.y;
+    const int c = 2 * (blockIdx.x * 256 + threadIdx.x);
+    if (c >= cols) return;
+    const float* p = part + (size_t)t * cols + c;
+    float2 v = *(const float2*)p;
+#pragma unroll 4
+    for (int s = 1; s < slices; s++) {
+        const float2 u = *(const float2*)(p + s * slice_stride);
+        v.x = v.x + u.x;
+        v.y = v.y + u.y;
+    }
+    *(float2*)(y + (size_t)t * ld + c) = v;
 }
 
 hipError_t launch_dequant_rows(int type, const void* w, int stride, int rows, int n, float* dst, hipStream_t s) {
@@ -415,23 +441,54 @@ struct SplitBufs {
     _Float16* x3;
     float* x_inv;
     float* y;
-    float* image;  // of X, for the reference-order projection (image_floats, 0: none)
+    float* parts;  // the GEMM's K slices, where they are summed into y
+    float* image;  // of X, for the reference-order projection
 };
 
-static size_t split_need(int n_tok, int n, size_t total, size_t image) {
-    return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2) + up256((size_t)n_tok * 4) + up256((size_t)n_tok * total * 4) +
-           image * 4;
+// Bytes of one batched product's buffers: y_floats of result, part_floats of K
+// slices and an image of image floats.
+static size_t split_need(int n_tok, int n, size_t y_floats, size_t part_floats, size_t image) {
+    return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2) + up256((size_t)n_tok * 4) + up256(y_floats * 4) +
+           up256(part_floats * 4) + image * 4;
 }
 
-static int ensure_split(pqa_ctx* ctx, int n_tok, int n, size_t total, size_t image, SplitBufs* sb, const char* fn) {
-    const size_t xb = up256((size_t)n_tok * 2 * pqa::k_half(n) * 2), xs = up256((size_t)n_tok * 4);
-    if (int rc = grow_split(ctx, split_need(n_tok, n, total, image), fn)) return rc;
+static int ensure_split(pqa_ctx* ctx, int n_tok, int n, size_t y_floats, size_t part_floats, size_t image,
+                        SplitBufs* sb, const char* fn) {
+    if (int rc = grow_split(ctx, split_need(n_tok, n, y_floats, part_floats, image), fn)) return rc;
     char* base = (char*)ctx->bsplit;
     sb->x3 = (_Float16*)base;
-    sb->x_inv = (float*)(base + xb);
-    sb->y = (float*)(base + xb + xs);
-    sb->image = (float*)(base + xb + xs + up256((size_t)n_tok * total * 4));
+    base += up256((size_t)n_tok * 2 * pqa::k_half(n) * 2);
+    sb->x_inv = (float*)base;
+    base += up256((size_t)n_tok * 4);
+    sb->y = (float*)base;
+    base += up256(y_floats * 4);
+    sb->parts = (float*)base;
+    base += up256(part_floats * 4);
+    sb->image = (float*)base;
     return PQA_OK;
+}
+
+// The buffers of the q/k/v product (q_only: the GEMM covers the q columns alone
+// and the reference-order projection needs an image) and of the output product.
+struct BatchShape {
+    pqa::GemmPlan plan;
+    size_t y_floats, part_floats, image;
+};
+static BatchShape qkv_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok, bool q_only) {
+    const size_t total = ctx->q_dim + 2 * ctx->kv_dim, cols = q_only ? ctx->q_dim : total;
+    BatchShape b;
+    b.plan = pqa::gemm_f16x3_plan(n_tok, (int)cols, pqa::k_half(p.n_embd), ctx->cu_count);
+    b.y_floats = (size_t)n_tok * total;
+    b.part_floats = b.plan.slices > 1 ? (size_t)b.plan.slices * n_tok * cols : 0;
+    b.image = q_only ? image_floats(p, n_tok) : 0;
+    return b;
+}
+static BatchShape out_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok) {
+    BatchShape b;
+    b.plan = pqa::gemm_f16x3_plan(n_tok, p.out_rows, pqa::k_half((int)ctx->q_dim), ctx->cu_count);
+    b.y_floats = (size_t)b.plan.slices * n_tok * p.out_rows;  // the residual kernel sums the slices
+    b.part_floats = b.image = 0;
+    return b;
 }
 
 // X' and the GEMM of one call: sb->y [n_tok][q_dim + 2 kv_dim] = X W^T, every
@@ -447,15 +504,22 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
     const int kh = pqa::k_half(n);
     const _Float16* w3 = (const _Float16*)p.split;
     *w_inv = (const float*)((const char*)p.split + up256(total * 2 * kh * 2));
-    if (int rc = ensure_split(ctx, n_tok, n, total, q_only ? image_floats(p, n_tok) : 0, sb, fn)) return rc;
+    const BatchShape bs = qkv_shape(ctx, p, n_tok, q_only);
+    if (int rc = ensure_split(ctx, n_tok, n, bs.y_floats, bs.part_floats, bs.image, sb, fn)) return rc;
     pqa::launch_split2(xb, n_tok, n, sb->x3, kh, sb->x_inv, ctx->stream);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
     // Y[n_tok][total] = X_hi W_hi^T + X_hi W_lo^T + X_lo W_hi^T (the q rows come first)
-    const int ncols = q_only ? (int)ctx->q_dim : (int)total;
-    return hip_check(ctx,
-                     pqa::launch_gemm_f16x3_nt(sb->x3, 2 * kh, w3, 2 * kh, sb->y, (int)total, n_tok, ncols, kh,
-                                                        ctx->stream),
-                     fn);
+    const int cols = q_only ? (int)ctx->q_dim : (int)total;
+    const bool sliced = bs.plan.slices > 1;
+    const size_t stride = (size_t)n_tok * cols;
+    const hipError_t e =
+        pqa::launch_gemm_f16x3_nt(bs.plan, sb->x3, 2 * kh, w3, 2 * kh, sliced ? sb->parts : sb->y,
+                                  sliced ? cols : (int)total, stride, n_tok, cols, kh, ctx->stream);
+    if (int rc = hip_check(ctx, e, fn)) return rc;
+    if (sliced)
+        hipLaunchKernelGGL(pqa::sum_slices_kernel, dim3((cols / 2 + 255) / 256, n_tok), dim3(256), 0, ctx->stream,
+                           (const float*)sb->parts, bs.plan.slices, stride, cols, sb->y, (int)total);
+    return hip_check(ctx, hipGetLastError(), fn);
 }
 
 static int check_batch(pqa_ctx* ctx, int layer, int n_tok, const char* fn) {
@@ -546,20 +610,23 @@ static int out_project_batch(pqa_ctx* ctx, int layer, int n_tok, const float* at
     const auto& p = ctx->proj[layer];
     const int n = (int)ctx->q_dim, rows = p.out_rows;
     const int kh = pqa::k_half(n);
+    const BatchShape bs = out_shape(ctx, p, n_tok);
     SplitBufs sb;
-    if (int rc = ensure_split(ctx, n_tok, n, (size_t)rows, 0, &sb, fn)) return rc;
+    if (int rc = ensure_split(ctx, n_tok, n, bs.y_floats, 0, 0, &sb, fn)) return rc;
     pqa::launch_split2(attn, n_tok, n, sb.x3, kh, sb.x_inv, ctx->stream);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
     const _Float16* w3 = (const _Float16*)p.out_split;
     const float* w_inv = (const float*)((const char*)p.out_split + up256((size_t)rows * 2 * kh * 2));
+    const size_t stride = (size_t)n_tok * rows;
     if (int rc = hip_check(ctx,
-                           pqa::launch_gemm_f16x3_nt(sb.x3, 2 * kh, w3, 2 * kh, sb.y, rows, n_tok, rows, kh,
-                                                     ctx->stream),
+                           pqa::launch_gemm_f16x3_nt(bs.plan, sb.x3, 2 * kh, w3, 2 * kh, sb.y, rows, stride, n_tok,
+                                                     rows, kh, ctx->stream),
                            fn))
         return rc;
     const unsigned gx = (unsigned)((rows / 4 + 255) / 256);
     hipLaunchKernelGGL(pqa::unscale_residual_kernel, dim3(gx, n_tok), dim3(256), 0, ctx->stream, (const float*)sb.y,
-                       rows, w_inv, (const float*)sb.x_inv, (const uint8_t*)p.b[3], p.btype[3], x);
+                       bs.plan.slices, stride, rows, w_inv, (const float*)sb.x_inv, (const uint8_t*)p.b[3],
+                       p.btype[3], x);
     return hip_check(ctx, hipGetLastError(), fn);
 }
 
@@ -595,10 +662,9 @@ extern "C" int pqa_prefill_block(pqa_ctx* ctx, int layer, int start_pos, int n_t
         return set_err(ctx, PQA_ERR_RANGE, "pqa_prefill_block: positions past max_seq_len");
     // every buffer of both GEMMs exists before the first kernel is queued
     const auto& p = ctx->proj[layer];
-    const size_t total = ctx->q_dim + 2 * ctx->kv_dim;
-    const size_t image = ctx->batch_exact_kv ? image_floats(p, n_tok) : 0;
-    const size_t need =
-        std::max(split_need(n_tok, p.n_embd, total, image), split_need(n_tok, (int)ctx->q_dim, p.out_rows, 0));
+    const BatchShape bq = qkv_shape(ctx, p, n_tok, ctx->batch_exact_kv != 0), bo = out_shape(ctx, p, n_tok);
+    const size_t need = std::max(split_need(n_tok, p.n_embd, bq.y_floats, bq.part_floats, bq.image),
+                                 split_need(n_tok, (int)ctx->q_dim, bo.y_floats, 0, 0));
     if (int rc = grow_split(ctx, need, fn)) return rc;
     const size_t af = (size_t)n_tok * ctx->q_dim;
     if (af > ctx->battn_floats) {

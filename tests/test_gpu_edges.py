@@ -42,3 +42,41 @@ def test_ordered_projection_tile_edges(n_tok, kt, vt, dim):
     for name, g, j in (("k", k, 1), ("v", v, 2)):
         assert_bits_equal(_bits(g), _bits(O.matmul_bias_tokens(x, w[j], types[j], rows[j], b[j], bt[j])), name)
     att.close()
+
+
+# the split GEMM's workgroup tiles (64 to 256 rows, 64 to 192 columns, with and without K
+# slices): token counts around the tile edges, widths whose K is one, an odd number and many
+# 32-wide tiles, and columns that leave partial tiles
+@pytest.mark.parametrize("n_tok,dim,nh", [(1, 8, 3), (63, 40, 3), (65, 1000, 3), (128, 2048, 16), (129, 896, 14),
+                                          (257, 1032, 32), (513, 2560, 32), (1025, 512, 44)])
+def test_split_gemm_tile_edges(n_tok, dim, nh):
+    print(f"split GEMM, {n_tok} tokens, width {dim}, {nh} heads", flush=True)
+    rng = np.random.default_rng(7 * n_tok + dim)
+    nkv, hd, wt = 1, 64, O.GGUF_F32
+    att = PicoAttention(1, 16, nh, nkv, hd)
+    rows = (nh * hd, hd, hd)
+    w = [make_rows(rng, wt, r, dim) for r in rows]
+    b = make_bias(rng, O.GGUF_F32, rows[0])
+    att.set_qkv_weights(0, dim, w[0], wt, w[1], wt, w[2], wt, b, O.GGUF_F32)
+    wo, bo = make_rows(rng, wt, 4 * dim, nh * hd), make_bias(rng, O.GGUF_F32, 4 * dim)
+    att.set_out_weights(0, 4 * dim, wo, wt, bo, O.GGUF_F32)
+    x = rng.standard_normal((n_tok, dim)).astype(np.float32)
+    wf = [m.view(np.float32).astype(np.float64) for m in (*w, wo)]
+    # 3 n products of 22-bit operands: within (3 n + 12) 2^-24 sum |w x| of the exact sum, and a
+    # rounding of the bias sum (and of the residual sum) on top
+    for exact_kv in (False, True):
+        att.set_batch_projection(exact_kv)
+        got = [g.cpu().numpy().astype(np.float64) for g in att.qkv_project_batch(0, torch.from_numpy(x).to(DEV))]
+        for j in range(1 if exact_kv else 3):
+            want = x.astype(np.float64) @ wf[j].T + (b.view(np.float32) if j == 0 else 0.0)
+            mag = np.abs(x.astype(np.float64)) @ np.abs(wf[j]).T
+            assert np.all(np.abs(got[j] - want) <= (3 * dim + 12) * 2.0 ** -24 * mag + 2.0 ** -23 * np.abs(want) + 1e-30), j
+    a = rng.standard_normal((n_tok, nh * hd)).astype(np.float32)
+    x0 = rng.standard_normal((n_tok, 4 * dim)).astype(np.float32)
+    xo = torch.from_numpy(x0.copy()).to(DEV)
+    att.out_project_batch(0, torch.from_numpy(a).to(DEV), xo)
+    y = a.astype(np.float64) @ wf[3].T + bo.view(np.float32)
+    mag = np.abs(a.astype(np.float64)) @ np.abs(wf[3]).T
+    tol = (3 * nh * hd + 12) * 2.0 ** -24 * mag + 2.0 ** -23 * (np.abs(y) + np.abs(y + x0)) + 1e-30
+    assert np.all(np.abs(xo.cpu().numpy() - (y + x0)) <= tol)
+    att.close()
