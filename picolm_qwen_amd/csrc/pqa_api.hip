@@ -36,8 +36,7 @@ static void free_ctx(pqa_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     pqa_free_projections(c);
     pqa_free_batch(c);
-    void* bufs[] = {c->key_cache, c->val_cache, c->rope_cos, c->rope_sin, c->qk_norm, c->part_acc,
-                    c->part_ml,   c->stage,     c->qkv,      c->gen_q};
+    void* bufs[] = {c->key_cache, c->val_cache, c->slab, c->stage, c->gen_q};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->hstage) (void)hipHostFree(c->hstage);
@@ -109,16 +108,32 @@ extern "C" int pqa_create(pqa_ctx** out, int n_layers, int max_seq_len, int n_he
         chk(hipMemset(c->key_cache, 0, cache * 2), "memset");
         chk(hipMemset(c->val_cache, 0, cache * 2), "memset");
     }
-    if (chk(dev_alloc(&c->rope_cos, (size_t)max_seq_len * half), "rope") &&
-        chk(dev_alloc(&c->rope_sin, (size_t)max_seq_len * half), "rope")) {
+    // one allocation for the rest: each costs a context's user as much as megabytes of it
+    const bool mfma = pqa::mfma_head_dim(head_dim);
+    if (mfma)  // two rounds of one 128-row block per CU, at most 16 ranges of every row there can be
+        c->pf_rows = std::min<size_t>((size_t)c->cu_count * 256, (size_t)max_seq_len * n_heads * 16);
+    const struct {
+        float** p;
+        size_t floats;
+    } parts[] = {{&c->rope_cos, (size_t)max_seq_len * half},
+                 {&c->rope_sin, (size_t)max_seq_len * half},
+                 {&c->qk_norm, (size_t)n_layers * 2 * head_dim},
+                 {&c->part_acc, (size_t)ny * c->max_splits * c->chunk_heads * head_dim},
+                 {&c->part_ml, (size_t)ny * c->max_splits * c->chunk_heads * 2},
+                 {&c->qkv, 2 * c->q_dim + 2 * c->kv_dim},
+                 {&c->pf_part, c->pf_rows * (head_dim + 2)}};
+    size_t slab = 0;
+    for (const auto& part : parts) slab += (part.floats * sizeof(float) + 255) & ~(size_t)255;
+    if (chk(dev_alloc(&c->slab, slab), "tables and workspaces")) {
+        size_t off = 0;
+        for (const auto& part : parts) {
+            *part.p = (float*)(c->slab + off);
+            off += (part.floats * sizeof(float) + 255) & ~(size_t)255;
+        }
         chk(hipMemcpy(c->rope_cos, rope_cos, (size_t)max_seq_len * half * 4, hipMemcpyHostToDevice), "rope copy");
         chk(hipMemcpy(c->rope_sin, rope_sin, (size_t)max_seq_len * half * 4, hipMemcpyHostToDevice), "rope copy");
     }
-    chk(dev_alloc(&c->qk_norm, (size_t)n_layers * 2 * head_dim), "qk norm");
-    chk(dev_alloc(&c->part_acc, (size_t)ny * c->max_splits * c->chunk_heads * head_dim), "workspace");
-    chk(dev_alloc(&c->part_ml, (size_t)ny * c->max_splits * c->chunk_heads * 2), "workspace");
-    chk(dev_alloc(&c->qkv, 2 * c->q_dim + 2 * c->kv_dim), "workspace");
-    if (!pqa::mfma_head_dim(head_dim) && chk(dev_alloc(&c->gen_q, c->q_dim), "workspace")) c->gen_q_floats = c->q_dim;
+    if (!mfma && chk(dev_alloc(&c->gen_q, c->q_dim), "workspace")) c->gen_q_floats = c->q_dim;
     if (rc == PQA_OK) {
         // the no-allocation decode's scratch address on this device
         const int src = pqa::scratch_init(c->device);

@@ -61,6 +61,16 @@ struct pqa_ctx {
     int split_override = 0;
     int cu_count = 256;
 
+    // prefill partials of key ranges: [pf_rows][head_dim] floats, then
+    // [pf_rows][2]; made with the context, so that a prefill allocates nothing
+    // and captured launches keep a valid address
+    float* pf_part = nullptr;
+    size_t pf_rows = 0;
+
+    // one allocation for the tables and workspaces whose size the context's
+    // shape fixes: rope_cos to pf_part point into it
+    char* slab = nullptr;
+
     // prefill: q = fp16 hi + lo in the score products (outlier-heavy caches)
     // prefill q: 1 (default) fp16 hi + lo, fp32-level scores; 0 one fp16 q,
     // whose score error grows with |q| |k|

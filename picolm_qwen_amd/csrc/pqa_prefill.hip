@@ -28,6 +28,7 @@
 //    loads, double buffered, one barrier per tile pair; V fragments are read
 //    with transposing LDS reads. Tiles past the causal limit of every row in
 //    a wave are skipped. Outputs leave through LDS as whole 512-byte rows.
+#include <algorithm>
 #include <type_traits>
 
 #include "pqa_device.h"
@@ -236,6 +237,12 @@ struct AttnArgs {
     const float* x_inv;
     const uint8_t* qb;
     int qbt;
+    // RANGES: key ranges per row block; with more than one, range s of row R
+    // leaves its unnormalised output at part + (s n_tok nh + output row) HD and
+    // (maximum, sum) at part_ml + 2 (s n_tok nh + output row)
+    int nrange;
+    float* part;
+    float* part_ml;
 };
 
 // The prompt's q rows and output rows each cross the chip once: read and
@@ -280,7 +287,10 @@ struct PrefillTile {
 
 // SPLITQ: scores use q = hi + lo (two fp16 MFMAs into one fp32 accumulator),
 // which keeps fp32-level score precision when keys carry large outliers.
-template <int HD, bool SPLITQ, bool YS>
+// RANGES: a workgroup takes one row block and one of nrange ranges of its key
+// tiles instead of a pair of blocks (prompts whose pairs leave CUs idle, see
+// prefill_ranges); prefill_combine_kernel merges the ranges.
+template <int HD, bool SPLITQ, bool YS, bool RANGES>
 __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const AttnArgs a) {
     using T = PrefillTile<HD>;
     constexpr int KS = HD / 32;  // 32-dim k-steps of S^T = K Q^T
@@ -301,8 +311,9 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
     // head's K/V in one L2. Inside the workgroup the two waves of a SIMD
     // (w and w + 4) own the same rows and alternate key tiles: equal work.
     const int kvh = (int)blockIdx.x % a.n_kv;
-    const int pair = (int)blockIdx.x / a.n_kv;
-    const int nb = a.nblk - 1 - pair == pair ? 1 : 2;
+    const int pair = RANGES ? (int)blockIdx.x / a.n_kv / a.nrange : (int)blockIdx.x / a.n_kv;
+    const int range = RANGES ? (int)blockIdx.x / a.n_kv - pair * a.nrange : 0;
+    const int nb = RANGES || a.nblk - 1 - pair == pair ? 1 : 2;
 
     const char* kbase = (const char*)(a.kc + (size_t)kvh * HD);
     const char* vbase = (const char*)(a.vc + (size_t)kvh * HD);
@@ -369,12 +380,15 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
         for (int rb = 0; rb < 2; rb++) qpos[rb] = a.start + min(R0 + 16 * rb + c16, a.rows - 1) / a.g;
         const int last_row_blk = min(a.rows, (b + 1) * kRowsPerBlock) - 1;
         const int kend = a.start + last_row_blk / a.g + 1;
-        const int ntiles = (kend + kKeysPerTile - 1) / kKeysPerTile;
+        const int ktiles = (kend + kKeysPerTile - 1) / kKeysPerTile;
+        // key tiles [tile0, ntiles) of this workgroup
+        const int tile0 = RANGES ? (int)((long long)ktiles * range / a.nrange) : 0;
+        const int ntiles = RANGES ? (int)((long long)ktiles * (range + 1) / a.nrange) : ktiles;
         const int kend_w = R0 < a.rows ? a.start + (min(a.rows, R0 + 32) - 1) / a.g + 1 : 0;
         const int qpos_min_w = R0 < a.rows ? a.start + R0 / a.g : 0;
 
         auto issue = [&](int step, int buf) {
-            const int kt = 2 * step + par;
+            const int kt = tile0 + 2 * step + par;
             if (kt >= ntiles) return;
             const int key0 = kt * kKeysPerTile;
             const char* kb = kbase + (size_t)key0 * rowb;
@@ -587,7 +601,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
 
         auto tile = [&](int step, auto BUF) {
             constexpr int buf = decltype(BUF)::value;
-            const int kt = 2 * step + par;
+            const int kt = tile0 + 2 * step + par;
             const int key0 = kt * kKeysPerTile;
             PQA_SSTAMP(step, kSStStart);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of step `step`
@@ -756,7 +770,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
             PQA_SSTAMP(step, kSStPV);
         };
 
-        const int nsteps = (ntiles + 1) / 2;
+        const int nsteps = (ntiles - tile0 + 1) / 2;
         for (int step = 0; step < nsteps; step += 2) {
             tile(step, std::integral_constant<int, 0>{});
             if (step + 1 < nsteps) tile(step + 1, std::integral_constant<int, 1>{});
@@ -804,7 +818,9 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
             const float M = fmaxf(me, mo);
             const float fe = fast_exp2(me - M);
             const float fo = fast_exp2(mo - M);
-            const float inv = 1.0f / sum_x32(sum_x16(fmaf(le, fe, lo * fo)));
+            const float lsum = sum_x32(sum_x16(fmaf(le, fe, lo * fo)));
+            const bool partial = RANGES && a.nrange > 1;
+            const float inv = partial ? 1.0f : 1.0f / lsum;
             const float we = fe * inv, wo = fo * inv;
 #pragma unroll
             for (int db = 0; db < DB; db++)
@@ -831,6 +847,14 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
             // output row of q row 16 rbo + (lane & 15)
             const int Rl = R0 + 16 * rbo + c16;
             const int orow = Rl < a.rows ? (Rl / a.g) * a.nh + kvh * a.g + (Rl - (Rl / a.g) * a.g) : -1;
+            float* dst = a.out;
+            if constexpr (RANGES) {
+                if (partial) {
+                    const size_t first = (size_t)range * a.n_tok * a.nh;
+                    dst = a.part + first * HD;
+                    if (g16 == 0 && orow >= 0) *(float2*)(a.part_ml + 2 * (first + orow)) = float2{M, lsum};
+                }
+            }
             wave_sync();
             constexpr int RPS = 64 / CPR;          // rows per store instruction
             constexpr int NST = 16 * CPR / 64;     // store instructions per wave
@@ -850,8 +874,9 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
                     if (lane / CPR == u) orr = v;
                 }
                 if (orr >= 0) {
-                    if constexpr (kNtOut) __builtin_nontemporal_store(vv[i], (floatx4*)(a.out + (size_t)orr * HD + 4 * c));
-                    else *(floatx4*)(a.out + (size_t)orr * HD + 4 * c) = vv[i];
+                    // a range's partial is read again by the next launch
+                    if (kNtOut && !partial) __builtin_nontemporal_store(vv[i], (floatx4*)(dst + (size_t)orr * HD + 4 * c));
+                    else *(floatx4*)(dst + (size_t)orr * HD + 4 * c) = vv[i];
                 }
             }
         };
@@ -863,6 +888,71 @@ __global__ __launch_bounds__(kAttnThreads, 1) void prefill_attn_kernel(const Att
         else finish(std::integral_constant<int, 1>{});
         PQA_PSTAMP(32 * j + kPStStored + wr, lane == 0 && par == 0);
     }
+}
+
+// out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s over the key ranges of one
+// output row (a range past a row's keys has m = -1e30, weight 0). HD / 4 lanes
+// per row, all loads of four ranges in flight.
+template <int HD>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __restrict__ part,
+                                                              const float* __restrict__ part_ml, int rows, int nrange,
+                                                              float* __restrict__ out) {
+    constexpr int H4 = HD / 4;
+    const int row = (int)blockIdx.x * (256 / H4) + (int)threadIdx.x / H4;
+    const int c = threadIdx.x % H4;
+    if (row >= rows) return;
+    float M = -1e30f;
+#pragma unroll 4
+    for (int s = 0; s < nrange; s++) M = fmaxf(M, part_ml[2 * ((size_t)s * rows + row)]);
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float l = 0.0f;
+#pragma unroll 4
+    for (int s = 0; s < nrange; s++) {
+        const float2 ml = *(const float2*)(part_ml + 2 * ((size_t)s * rows + row));
+        const floatx4 o = *(const floatx4*)(part + ((size_t)s * rows + row) * HD + 4 * c);
+        const float w = fast_exp2(ml.x - M);
+        l = fmaf(w, ml.y, l);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] = fmaf(w, o[e], acc[e]);
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[e] *= inv;
+    __builtin_nontemporal_store(acc, (floatx4*)(out + (size_t)row * HD + 4 * c));
+}
+
+// Key ranges per row block, or 0: pairs of whole blocks (see prefill_attn_kernel).
+// Pairs give every workgroup the same causal work, which is best once they fill
+// the chip; a prompt with fewer blocks finishes sooner with a block per
+// workgroup, and behind a long history with its keys in ranges. The estimate
+// counts steps of two key tiles (1.9 us): a block's prologue and epilogue take
+// about 3, and ranges a second launch that reads their partials; the partials
+// may take max_rows output rows. Measured per layer (32 / 8 heads of 128), pairs
+// against ranges: 300 tokens at 12000 400 -> 95 + 5 us (3 ranges, 240 workgroups
+// for 40), 1000 at 8000 322 -> 219, 40 at 30000 958 -> 68; 75 tokens at 0, one
+// block per workgroup, 21 -> 11.5; 2048 at 0 stay in pairs.
+static int prefill_ranges(int start, int n_tok, int g, int n_kv, int nblk, int cu_count, size_t max_rows) {
+    auto rounds = [&](long long wgs) { return (double)((wgs + cu_count - 1) / cu_count); };
+    auto steps = [&](int b) {  // of block b
+        const int last = (int)std::min<long long>((long long)n_tok * g, (long long)(b + 1) * kRowsPerBlock) - 1;
+        return ((start + last / g) / kKeysPerTile + 2) / 2;
+    };
+    const double block = 3.0;
+    const int longest = steps(nblk - 1);
+    const double pair = nblk > 1 ? longest + steps(0) + 2 * block : longest + block;
+    double best = rounds((long long)(nblk + 1) / 2 * n_kv) * pair;
+    int ranges = 0;
+    const size_t rows = (size_t)n_tok * g * n_kv;
+    for (int s = 1; s <= 16 && s <= 2 * longest; s++) {
+        if (s > 1 && s * rows > max_rows) break;
+        const double combine = s > 1 ? 4.0 + s * (double)rows / 2e4 : 0.0;
+        const double t = rounds((long long)nblk * n_kv * s) * ((double)longest / s + block) + combine;
+        if (t < best) {
+            best = t;
+            ranges = s;
+        }
+    }
+    return ranges;
 }
 
 #ifdef PQA_PHASE_STAMPS
@@ -975,11 +1065,27 @@ static hipError_t launch_prefill_hd(pqa_ctx* ctx, int layer, int start, int n_to
         a.qb = ys->b[0];
         a.qbt = ys->bt[0];
     }
-    dim3 grid((a.nblk + 1) / 2 * ctx->n_kv_heads);  // pairs of row blocks
-    if (ctx->prefill_split_q)
-        hipLaunchKernelGGL((prefill_attn_kernel<HD, true, YS>), grid, dim3(kAttnThreads), 0, ctx->stream, a);
-    else
-        hipLaunchKernelGGL((prefill_attn_kernel<HD, false, YS>), grid, dim3(kAttnThreads), 0, ctx->stream, a);
+    a.n_tok = n_tok;
+    const int ranges = prefill_ranges(start, n_tok, a.g, a.n_kv, a.nblk, ctx->cu_count, ctx->pf_rows);
+    a.nrange = std::max(1, ranges);
+    a.part = ctx->pf_part;
+    a.part_ml = ctx->pf_part + ctx->pf_rows * HD;
+    const dim3 grid((ranges ? a.nblk * ranges : (a.nblk + 1) / 2) * ctx->n_kv_heads);
+#define PQA_PF(SQ, RG) \
+    hipLaunchKernelGGL((prefill_attn_kernel<HD, SQ, YS, RG>), grid, dim3(kAttnThreads), 0, ctx->stream, a)
+    if (ctx->prefill_split_q) {
+        if (ranges) PQA_PF(true, true);
+        else PQA_PF(true, false);
+    } else {
+        if (ranges) PQA_PF(false, true);
+        else PQA_PF(false, false);
+    }
+#undef PQA_PF
+    e = hipGetLastError();
+    if (e != hipSuccess || ranges < 2) return e;
+    const int orows = n_tok * ctx->n_heads, rpw = 256 / (HD / 4);
+    hipLaunchKernelGGL(prefill_combine_kernel<HD>, dim3((orows + rpw - 1) / rpw), dim3(256), 0, ctx->stream,
+                       (const float*)a.part, (const float*)a.part_ml, orows, ranges, out);
     return hipGetLastError();
 }
 

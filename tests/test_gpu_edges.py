@@ -80,3 +80,37 @@ def test_split_gemm_tile_edges(n_tok, dim, nh):
     tol = (3 * nh * hd + 12) * 2.0 ** -24 * mag + 2.0 ** -23 * (np.abs(y) + np.abs(y + x0)) + 1e-30
     assert np.all(np.abs(xo.cpu().numpy() - (y + x0)) <= tol)
     att.close()
+
+
+# prefill behind a history: blocks whose keys are cut into ranges (few blocks, a long history),
+# ranges past a row's own position, one block per workgroup without ranges, and prompts that
+# stay on block pairs; both head sizes, both q precisions
+@pytest.mark.parametrize("nh,nkv,hd,start,n_tok,split_q", [(4, 1, 64, 3000, 5, True), (2, 1, 128, 1000, 100, True),
+                                                           (7, 1, 64, 700, 65, False), (8, 2, 128, 2047, 1, True),
+                                                           (4, 2, 128, 64, 300, True), (32, 2, 64, 129, 700, True),
+                                                           (32, 1, 128, 500, 2100, False)])
+def test_prefill_key_ranges(nh, nkv, hd, start, n_tok, split_q):
+    print(f"prefill ranges {nh}/{nkv} x {hd}, {n_tok} tokens at {start}, split_q {split_q}", flush=True)
+    smax, seed, kvd = start + n_tok, 4100 + start, nkv * hd
+    cos, sin = O.rope_table(1e6, hd, smax)
+    att = PicoAttention(1, smax, nh, nkv, hd, 0, rope_cos=cos, rope_sin=sin)
+    att.set_prefill_precision(split_q)
+    att.synth_kv(0, 0, start, seed, 0.0)
+    kc, vc = np.zeros((smax, kvd), np.uint16), np.zeros((smax, kvd), np.uint16)
+    kc[:start], vc[:start] = O.synth_kv_rows(seed, 0, kvd, 0, start, 0.0)
+    q, k, v = O.batch_inputs(seed, 0, 0, n_tok, nh, nkv, hd)
+    out = att.forward_batch(0, start, *(torch.from_numpy(x).to(DEV) for x in (q, k, v))).cpu().numpy()
+    shp = O.shape(nh, nkv, hd, smax, 0)
+    qr = [O.append(shp, start + t, q[t], k[t], v[t], None, None, cos[start + t], sin[start + t], kc, vc)
+          for t in range(n_tok)]
+    gk, gv = att.kv_download(0, start, n_tok)
+    assert_bits_equal(gk, kc[start:], "K rows")
+    assert_bits_equal(gv, vc[start:], "V rows")
+    # P is rounded to fp16 for the PV product and its own sum (2^-11 each, relative to sum p |v|); one fp16 q
+    # moves a score by up to 2^-11 |q| |k| / sqrt(hd) (log2 units included), about 2^-8 at these N(0, 1) rows
+    rel = 2.0 ** -10 if split_q else 2.0 ** -6
+    for t in sorted({0, 1, n_tok // 2, n_tok - 2, n_tok - 1} & set(range(n_tok))):
+        want = O.attend_f64(shp, start + t, qr[t], kc, vc)
+        mag = O.attend_f64(shp, start + t, qr[t], kc, vc & 0x7FFF)
+        assert np.all(np.abs(out[t] - want) <= rel * mag + 1e-6), t
+    att.close()
