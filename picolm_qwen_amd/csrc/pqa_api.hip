@@ -109,9 +109,10 @@ extern "C" int pqa_create(pqa_ctx** out, int n_layers, int max_seq_len, int n_he
         chk(hipMemset(c->val_cache, 0, cache * 2), "memset");
     }
     // one allocation for the rest: each costs a context's user as much as megabytes of it
-    const bool mfma = pqa::mfma_head_dim(head_dim);
-    if (mfma)  // two rounds of one 128-row block per CU, at most 16 ranges of every row there can be
-        c->pf_rows = std::min<size_t>((size_t)c->cu_count * 256, (size_t)max_seq_len * n_heads * 16);
+    const bool mfma = pqa::mfma_head_dim(head_dim), gen_mma = pqa::gen_mma_head_dim(head_dim);
+    // two rounds of one row block (128 rows, 64 on the general path) per CU, at most 16 ranges of every row there can be
+    if (mfma || gen_mma)
+        c->pf_rows = std::min<size_t>((size_t)c->cu_count * (mfma ? 256 : 128), (size_t)max_seq_len * n_heads * 16);
     const struct {
         float** p;
         size_t floats;
@@ -133,7 +134,7 @@ extern "C" int pqa_create(pqa_ctx** out, int n_layers, int max_seq_len, int n_he
         chk(hipMemcpy(c->rope_cos, rope_cos, (size_t)max_seq_len * half * 4, hipMemcpyHostToDevice), "rope copy");
         chk(hipMemcpy(c->rope_sin, rope_sin, (size_t)max_seq_len * half * 4, hipMemcpyHostToDevice), "rope copy");
     }
-    if (!mfma && chk(dev_alloc(&c->gen_q, c->q_dim), "workspace")) c->gen_q_floats = c->q_dim;
+    if (!mfma && !gen_mma && chk(dev_alloc(&c->gen_q, c->q_dim), "workspace")) c->gen_q_floats = c->q_dim;
     if (rc == PQA_OK) {
         // the no-allocation decode's scratch address on this device
         const int src = pqa::scratch_init(c->device);

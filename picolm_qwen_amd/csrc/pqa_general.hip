@@ -1,6 +1,8 @@
-// Attention for the head sizes the MFMA kernels are not built for: any even
-// head_dim up to 512 (cpp/model.hpp:172 sizes its accumulator for 512), for
-// decode and prefill alike.
+// Attention for the head sizes without kernels of their own: any even head_dim
+// up to 512 (cpp/model.hpp:172 sizes its accumulator for 512), for decode and
+// prefill alike. The sizes that models use go on to the MFMA kernels of
+// pqa_general_mma.hip (a prompt's K and V rows are appended here); the others
+// run on the kernels below.
 //
 // Two launches (three with splits):
 //   gen_prep_kernel  one wave per (token, head): the head's q or k through
@@ -19,8 +21,7 @@
 // LDS-tiled operand path, which is what the 64/128 kernels add.
 #include <algorithm>
 
-#include "pqa_device.h"
-#include "pqa_internal.h"
+#include "pqa_general.h"
 
 namespace pqa {
 
@@ -28,26 +29,6 @@ constexpr int kGenMaxHd = 512;
 constexpr int kMaxGenSplits = 256;  // the combine keeps one weight per key range in LDS
 constexpr int kGenWaves = 4;
 constexpr int kGenMaxG = 8;  // query heads per wave (a KV head's chunk)
-
-// One q/k/v operand: column c of token t at p[t * ld + c]; with w_inv the
-// value is the batched GEMM's scaled result, p * (w_inv[c] * x_inv[t]) + b[c].
-struct GenSrc {
-    const float* p;
-    int ld;
-    const float* w_inv;
-    const float* x_inv;
-    const uint8_t* b;
-    int bt;
-};
-
-__device__ __forceinline__ float gen_load(const GenSrc& s, int t, int c) {
-    float v = s.p[(size_t)t * s.ld + c];
-    if (s.w_inv) {
-        v = v * (s.w_inv[c] * s.x_inv[t]);
-        if (s.b) v = v + (s.bt == GG_F32 ? ((const float*)s.b)[c] : f16_bits_to_f32(((const uint16_t*)s.b)[c]));
-    }
-    return v;
-}
 
 struct GenPrepArgs {
     GenSrc q, k, v;
@@ -63,7 +44,8 @@ struct GenPrepArgs {
 };
 
 // grid (ceil((nh + nkv) / 4), n_tok); wave -> one head of one token (query
-// heads first, then KV heads, which also write their V row).
+// heads first, then KV heads, which also write their V row; nh = 0: the KV heads
+// alone).
 __global__ __launch_bounds__(64 * kGenWaves) void gen_prep_kernel(const GenPrepArgs a) {
     __shared__ float s_row[kGenWaves][kGenMaxHd];
     const int lane = threadIdx.x & 63;
@@ -475,7 +457,7 @@ static hipError_t ensure_gen_q(pqa_ctx* ctx, size_t floats) {
 }
 
 static hipError_t launch_gen_prep(pqa_ctx* ctx, int layer, int start, int n_tok, const GenSrc& q, const GenSrc& k,
-                                  const GenSrc& v) {
+                                  const GenSrc& v, bool with_q) {
     const int hd = ctx->head_dim;
     GenPrepArgs p;
     p.q = q;
@@ -491,12 +473,12 @@ static hipError_t launch_gen_prep(pqa_ctx* ctx, int layer, int start, int n_tok,
     p.qp = ctx->gen_q;
     p.start = start;
     p.n_tok = n_tok;
-    p.nh = ctx->n_heads;
+    p.nh = with_q ? ctx->n_heads : 0;
     p.nkv = ctx->n_kv_heads;
     p.hd = hd;
     p.rope = ctx->rope_style;
     p.qscale = 1.4426950408889634f / sqrtf((float)hd);
-    const int heads = ctx->n_heads + ctx->n_kv_heads;
+    const int heads = p.nh + ctx->n_kv_heads;
     hipLaunchKernelGGL(gen_prep_kernel, dim3((heads + kGenWaves - 1) / kGenWaves, n_tok), dim3(64 * kGenWaves), 0,
                        ctx->stream, p);
     return hipGetLastError();
@@ -567,17 +549,22 @@ static GenSrc plain_src(const float* p, size_t ld) { return GenSrc{p, (int)ld, n
 
 hipError_t launch_decode_general(pqa_ctx* ctx, int layer, int pos, const float* q, const float* k, const float* v,
                                  float* out, const DecodeWorkspace& ws) {
+    if (gen_mma_head_dim(ctx->head_dim))
+        return launch_gen_mma(ctx, layer, pos, 1, true, plain_src(q, ctx->q_dim), plain_src(k, ctx->kv_dim),
+                              plain_src(v, ctx->kv_dim), out, ws.part_acc, ws.part_ml,
+                              (size_t)ws.max_splits * ctx->n_heads);
     // gen_q holds one token's q from context creation on: no allocation here
     if (ctx->gen_q_floats < ctx->q_dim) return hipErrorInvalidValue;
     hipError_t e = launch_gen_prep(ctx, layer, pos, 1, plain_src(q, ctx->q_dim), plain_src(k, ctx->kv_dim),
-                                   plain_src(v, ctx->kv_dim));
+                                   plain_src(v, ctx->kv_dim), true);
     if (e != hipSuccess) return e;
     return launch_gen_attn(ctx, layer, pos, 1, out, &ws);
 }
 
 hipError_t launch_prefill_general(pqa_ctx* ctx, int layer, int start, int n_tok, const float* q, const float* k,
                                   const float* v, const PrefillScaled* ys, float* out) {
-    hipError_t e = ensure_gen_q(ctx, (size_t)n_tok * ctx->q_dim);
+    const bool mma = gen_mma_head_dim(ctx->head_dim);
+    hipError_t e = mma ? hipSuccess : ensure_gen_q(ctx, (size_t)n_tok * ctx->q_dim);
     if (e != hipSuccess) return e;
     GenSrc sq, sk, sv;
     if (ys) {
@@ -591,8 +578,11 @@ hipError_t launch_prefill_general(pqa_ctx* ctx, int layer, int start, int n_tok,
         sk = plain_src(k, ctx->kv_dim);
         sv = plain_src(v, ctx->kv_dim);
     }
-    e = launch_gen_prep(ctx, layer, start, n_tok, sq, sk, sv);
+    e = launch_gen_prep(ctx, layer, start, n_tok, sq, sk, sv, !mma);
     if (e != hipSuccess) return e;
+    if (mma)
+        return launch_gen_mma(ctx, layer, start, n_tok, false, sq, sk, sv, out, ctx->pf_part,
+                              ctx->pf_part + ctx->pf_rows * ctx->head_dim, ctx->pf_rows);
     return launch_gen_attn(ctx, layer, start, n_tok, out, nullptr);
 }
 

@@ -1,0 +1,684 @@
+// Attention at the head sizes 80, 96, 112, 160, 192 and 256 on the matrix cores,
+// for decode and prefill alike; the contracts are those of pqa_general.hip, whose
+// VALU kernels keep the other sizes (one wave per token and KV head there, bound
+// by load latency and by 2 fp32 operations per key, head and dim).
+//
+// The general path computes in fp32, so every operand that is not an fp16 cache
+// value is split into two fp16 parts with 22 significant bits together: q hi + lo
+// (each row first scaled by a power of two so that its largest element lies in
+// [2^14, 2^15)) against K, and P = exp2(score - max + 6) hi + lo against V, both
+// sums in fp32. Rows (query heads of one KV head, token by token) are packed 16 to
+// a wave: S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, in whose
+// layouts a lane's scores are already its operand of the second product. A last
+// half k-step of 16 dims (80, 112) takes v_mfma_f32_16x16x16_f16.
+//
+// K and V tiles of 64 keys (32 in a decode) arrive by direct global->LDS loads, 16-byte chunk c of
+// row r at slot c ^ x(r) (x within the largest power of two that divides the chunks
+// per row), free of bank conflicts for the K operand reads and the transposing V
+// reads alike.
+//   prefill  4 waves of 16 rows share each tile (two buffers, one barrier per
+//            tile);
+//   decode   the waves take a KV head's tiles in turn, each with two tiles of its
+//            own in flight behind the small operands; the wave with the last tile norms, rotates and rounds
+//            the new row, writes it to the cache and into its LDS tile. The waves'
+//            results meet in LDS.
+// Either may cut the keys into ranges (workgroups) whose partials gen_merge_kernel
+// combines.
+//
+// Measured per layer against the VALU kernels (launch count, all kernels): decode of
+// 32 / 8 heads of 96 at 9000 44 -> 22 us (13 us for the 27.6 MB of cache, merge 4;
+// the rest is the gap between two launches), 8 / 2 heads of 256 at 4 16 -> 6 us;
+// prefill of 700 tokens at head size 96 226 -> 41 us (kernel 207 -> 25; its bound is
+// the chain of one tile: operand reads, products, softmax, products), 851 at 256
+// 248 -> 46. The error against 64-bit sums is 0.6 to 0.8 times theirs.
+//
+// Infinities: a split product can turn inf into NaN (inf * 0, inf - inf), and a
+// masked key's V row still enters the product with weight 0. A row whose result is
+// not finite is therefore computed again by gen_row, with fp32 q, only its own
+// keys and no split.
+#include <algorithm>
+
+#include "pqa_general.h"
+
+namespace pqa {
+
+constexpr int kGmRows = 16;    // rows per wave
+constexpr float kGmSlack = 8.0f;  // log2 units between rescales: P stays <= 2^(8 + 6)
+constexpr float kGmShift = 6.0f;  // P is scaled by 2^6: its low part stays clear of fp16 subnormals
+
+struct GenMmaArgs {
+    GenSrc q, k, v;
+    const float* qn;  // [hd] or null
+    const float* kn;
+    const float* cos_tab;  // [S][hd / 2]
+    const float* sin_tab;
+    uint16_t* kc;  // the layer's cache
+    uint16_t* vc;
+    float* out;       // [n_tok][nh * hd] with one range
+    float* part_acc;  // [nrange][n_tok * nh][hd]
+    float* part_ml;   // [nrange][n_tok * nh][2]
+    int start, n_tok, nh, g, n_kv, kv_dim, rope, rows, nblk, nrange;
+    int qvec, ovec;  // q / out rows may move as 16-byte vectors
+    float qscale;
+};
+
+__host__ __device__ constexpr int gm_pow2(int ch) { return ch % 16 == 0 ? 16 : ch % 8 == 0 ? 8 : ch % 4 == 0 ? 4 : ch % 2 == 0 ? 2 : 1; }
+
+template <int HD, int KEYS>
+struct GmTile {
+    static_assert(HD % 16 == 0 && HD <= 256, "head sizes of the MFMA kernels");
+    static constexpr int CH = HD / 8;                 // 16-byte chunks per row
+    static constexpr int ROWB = HD * 2;
+    static constexpr int BYTES = KEYS * ROWB;
+    static constexpr int NI = BYTES / 1024;           // 1 KB loads per operand
+    static constexpr int P2 = gm_pow2(CH);
+    static constexpr int PER = 16 / P2;               // rows after which the bank of a chunk repeats
+    __device__ static int xk(int r) { return (r / PER) & (P2 - 1); }
+    __device__ static int xv(int r) { return (2 * (r / PER)) & (P2 - 1); }
+};
+
+// waves of a decode workgroup: two tiles each within the LDS
+template <int HD>
+constexpr int gm_decode_waves() { return HD <= 128 ? 4 : 2; }
+
+// keys per tile: 64 in a prefill (a tile of 32 is one dependent chain of short
+// products, 1.1 us at head size 96) unless two of them and the q rows exceed the
+// LDS; 32 in a decode, whose waves have two tiles each
+template <int HD, bool DECODE>
+constexpr int gm_keys() { return DECODE || HD > 192 ? 32 : 64; }
+
+__device__ __forceinline__ float4 gm_load4(const GenSrc& s, int t, int c, int vec) {
+    if (s.w_inv || !vec) return float4{gen_load(s, t, c), gen_load(s, t, c + 1), gen_load(s, t, c + 2), gen_load(s, t, c + 3)};
+    return *(const float4*)(s.p + (size_t)t * s.ld + c);
+}
+
+// The row at q (fp32, prepared) over the keys of tiles first, first + step, ...
+// below end that are at most qpos, in fp32: m, l and the accumulator (row acc, may
+// alias q) in the scale of the MFMA path. One wave.
+template <int HD, int KEYS>
+__device__ void gen_row(const uint16_t* kbase, const uint16_t* vbase, size_t stride, const float* q, int qpos, int first,
+                        int step, int end, int lane, float* acc_row, float& m_out, float& l_out) {
+    constexpr int NA = (HD + 63) / 64;
+    float m = -1e30f, l = 0.0f, acc[NA];
+#pragma unroll
+    for (int i = 0; i < NA; i++) acc[i] = 0.0f;
+    for (int kt = first; kt < end; kt += step) {
+        const int key0 = kt * KEYS, nk = min(KEYS, qpos + 1 - key0);
+        if (nk <= 0) break;
+        const bool valid = lane < nk;
+        const u32x4* kr = (const u32x4*)(kbase + (size_t)(key0 + (valid ? lane : 0)) * stride);
+        float s = 0.0f;
+        for (int c = 0; c < HD / 8; c++) {
+            const u32x4 u = kr[c];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                s = fmaf(q[8 * c + 2 * e], f16_bits_to_f32((uint16_t)(u[e] & 0xFFFFu)), s);
+                s = fmaf(q[8 * c + 2 * e + 1], f16_bits_to_f32((uint16_t)(u[e] >> 16)), s);
+            }
+        }
+        const float sv = valid ? s : -__builtin_huge_valf();
+        const float mn = fmaxf(m, group_max<64>(sv));
+        const float corr = fast_exp2(m - mn);
+        const float p = valid ? fast_exp2(sv - mn + kGmShift) : 0.0f;
+        l = l * corr + group_sum<64>(p);
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < NA; i++) acc[i] *= corr;
+        for (int j = 0; j < nk; j++) {
+            const float pj = __shfl(p, j);
+            const uint16_t* vr = vbase + (size_t)(key0 + j) * stride;
+#pragma unroll
+            for (int i = 0; i < NA; i++) {
+                const int d = lane + 64 * i;
+                if (d < HD) acc[i] = fmaf(pj, f16_bits_to_f32(vr[d]), acc[i]);
+            }
+        }
+    }
+    wave_sync();  // q has been read
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+        if (lane + 64 * i < HD) acc_row[lane + 64 * i] = acc[i];
+    wave_sync();
+    m_out = m;
+    l_out = l;
+}
+
+// DECODE: one row group (16 query heads of one KV head at one token), waves on
+// different key tiles; else 4 row groups on the same tiles.
+template <int HD, bool DECODE>
+__global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen_mma_kernel(const GenMmaArgs a) {
+    constexpr int KEYS = gm_keys<HD, DECODE>(), KB = KEYS / 16;
+    using T = GmTile<HD, KEYS>;
+    constexpr int NW = DECODE ? gm_decode_waves<HD>() : 4;
+    constexpr int RW = DECODE ? 1 : 4, KW = NW / RW;  // row groups, key groups
+    constexpr int KS = HD / 32, DB = HD / 16;
+    constexpr bool HALF = HD % 32 != 0;
+    constexpr int QS = HD + 4;                        // LDS row stride of a q row
+    constexpr int NBUF = 2;
+    constexpr int LPW = (2 * T::NI + RW - 1) / RW;    // loads per wave and tile
+    constexpr int LPR = 4 * KW;                       // lanes per q row in its preparation
+    constexpr int D4 = HD / 4;
+    static_assert(!DECODE || kGmRows * QS * 4 <= 4 * T::BYTES, "a decode wave's result fits its tile buffers");
+    __shared__ __attribute__((aligned(1024))) char lds[KW][NBUF][2][T::BYTES];  // [key group][buffer][K, V]
+    __shared__ __attribute__((aligned(16))) float sq[RW][kGmRows * QS];  // prepared q; a prefill wave's result later
+    __shared__ float s_scale[RW][kGmRows];
+    __shared__ float s_ml[NW][2][kGmRows];
+    __shared__ __attribute__((aligned(16))) uint16_t s_new[2][DECODE ? HD : 8];
+    // decode: cos and sin [HD / 2] each, the norm weights of q and k, k and v
+    constexpr int ACOS = 0, ASIN = HD / 2, AQN = HD, AKN = 2 * HD, AK = 3 * HD, AV = 4 * HD;
+    __shared__ __attribute__((aligned(16))) float s_aux[DECODE ? 5 * HD : 4];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = w % RW, wk = w / RW;
+    const int c16 = lane & 15, g16 = lane >> 4;
+    const int kvh = (int)blockIdx.x % a.n_kv, rest = (int)blockIdx.x / a.n_kv;
+    const int blk = a.nblk - 1 - rest / a.nrange, range = rest % a.nrange;  // the longest blocks first
+    const int R0 = (blk * RW + wr) * kGmRows;
+    const int rlast = a.rows - 1;
+    const int last_blk = min(a.rows, (blk + 1) * RW * kGmRows) - 1;
+    const int kend = a.start + last_blk / a.g + 1;                    // keys of the block
+    const int klim = DECODE ? max(a.start, 1) : kend;                 // rows that are in the cache (row 0 exists)
+    const int ktiles = (kend + KEYS - 1) / KEYS;
+    const int tile0 = (int)((long long)ktiles * range / a.nrange) + wk;  // this wave's tiles: tile0, tile0 + KW, ...
+    const int tile1 = (int)((long long)ktiles * (range + 1) / a.nrange);
+    const size_t rowb = (size_t)a.kv_dim * 2;
+    const char* kbase = (const char*)(a.kc + (size_t)kvh * HD);
+    const char* vbase = (const char*)(a.vc + (size_t)kvh * HD);
+
+    // ---- K/V loads: piece pp of a tile is 1 KB load pp % NI of operand pp / NI;
+    // the row waves share the pieces (the last one may be loaded twice) ----
+    unsigned goff[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; i++) {
+        const int pp = min(wr + RW * i, 2 * T::NI - 1);
+        const int L = 64 * (pp % T::NI) + lane, r = L / T::CH;
+        goff[i] = (unsigned)(r * rowb) + 16u * (unsigned)((L % T::CH) ^ (pp < T::NI ? T::xk(r) : T::xv(r)));
+    }
+    auto issue = [&](int kt, int buf) __attribute__((always_inline)) {
+        if (kt >= tile1) return;
+        const int key0 = kt * KEYS;
+        const bool full = key0 + KEYS <= klim;
+        const int k0 = min(key0, klim - 1);  // a tile of the new row alone reads the row before it
+#pragma unroll
+        for (int i = 0; i < LPW; i++) {
+            const int pp = min(wr + RW * i, 2 * T::NI - 1);
+            unsigned off = goff[i];
+            if (!full) {  // rows past the last one repeat it (masked, or overwritten by the new row)
+                const int L = 64 * (pp % T::NI) + lane, r = L / T::CH;
+                off = (unsigned)(min(r, klim - 1 - k0) * rowb) +
+                      16u * (unsigned)((L % T::CH) ^ (pp < T::NI ? T::xk(r) : T::xv(r)));
+            }
+            const char* src = (pp < T::NI ? kbase : vbase) + (size_t)k0 * rowb;
+            lds_dma_b128(src, off, lds_addr(&lds[wk][buf][pp < T::NI ? 0 : 1][(pp % T::NI) * 1024]));
+        }
+    };
+    // ---- decode: q, k, v, the RoPE row and the norm weights go to LDS by direct
+    // loads too, ahead of the K/V tiles, so that the wave can wait for them alone
+    // (a wait the compiler places would cover the tiles in flight) ----
+    float* qreg = sq[wr];
+    const bool owner = DECODE && range == a.nrange - 1 && tile0 < tile1 && (tile1 - 1 - tile0) % KW == 0;
+    if constexpr (DECODE) {
+        auto fetch = [&](const float* src, int n, float* dst) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < (HD + 63) / 64; i++)
+                if (64 * i + lane < n) lds_dma_b32(src, 256u * i + 4u * lane, lds_addr(dst) + 256u * i);
+        };
+        const int nrow = min(kGmRows, rlast + 1 - R0);
+        const float* q0 = a.q.p + (size_t)(kvh * a.g + R0) * HD;
+        for (int r = wk; r < nrow; r += KW) fetch(q0 + (size_t)r * HD, HD, qreg + r * QS);
+        for (int r = nrow + wk; r < kGmRows; r += KW)
+            for (int e = lane; e < HD; e += 64) qreg[r * QS + e] = 0.0f;
+        const size_t rp = (size_t)a.start * (HD / 2);
+        if (wk == 0) {
+            fetch(a.cos_tab + rp, HD / 2, s_aux + ACOS);
+            fetch(a.sin_tab + rp, HD / 2, s_aux + ASIN);
+        }
+        if (wk == KW - 1 && a.qn) fetch(a.qn, HD, s_aux + AQN);
+        if (owner) {
+            if (a.kn) fetch(a.kn, HD, s_aux + AKN);
+            fetch(a.k.p + (size_t)kvh * HD, HD, s_aux + AK);
+            fetch(a.v.p + (size_t)kvh * HD, HD, s_aux + AV);
+        }
+    }
+    issue(tile0, 0);
+    if constexpr (DECODE) issue(tile0 + KW, 1);
+
+    // ---- q: normed, rotated, scaled, fp32 in LDS; its largest element's exponent ----
+    // Rows wk, wk + KW, ... of a decode's 16, the wave's own 16 in a prefill; LPR
+    // lanes each.
+    if constexpr (DECODE) {
+        const int mine = tile0 >= tile1 ? 0 : tile0 + KW >= tile1 ? 1 : 2;
+        if (mine == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW < 63 ? 2 * LPW : 63) : "memory");
+        else if (mine == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    {
+        const int pr = (lane / LPR) * KW + wk, sub = lane % LPR;
+        const int Rc = min(R0 + pr, rlast), tok = Rc / a.g;
+        const int col0 = (kvh * a.g + Rc - tok * a.g) * HD;
+        const bool live = R0 + pr <= rlast;
+        float* row = qreg + pr * QS;
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < (D4 + LPR - 1) / LPR; i++) {
+            const int f = sub + LPR * i;
+            if (f < D4) {
+                float4 x;
+                if constexpr (DECODE) {
+                    x = *(const float4*)(row + 4 * f);
+                } else {
+                    x = gm_load4(a.q, tok, col0 + 4 * f, a.qvec);
+                    if (!live) x = float4{0.0f, 0.0f, 0.0f, 0.0f};
+                    *(float4*)(row + 4 * f) = x;
+                }
+                ss = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, fmaf(x.w, x.w, ss))));
+            }
+        }
+        wave_sync();
+        float sc = a.qscale;
+        if (a.qn) sc = sc / sqrtf(group_sum<LPR>(ss) / (float)HD + 1e-6f);
+        const size_t half = HD / 2;
+        const float* cr = DECODE ? s_aux + ACOS : a.cos_tab + (size_t)(a.start + tok) * half;
+        const float* sr = DECODE ? s_aux + ASIN : a.sin_tab + (size_t)(a.start + tok) * half;
+        const float* qn = DECODE ? s_aux + AQN : a.qn;
+        float mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < (HD / 2 + LPR - 1) / LPR; i++) {
+            const int p = sub + LPR * i;
+            if (p < HD / 2) {
+                int e0, e1;
+                rope_pair(a.rope, p, HD, e0, e1);
+                float x0 = row[e0] * sc, x1 = row[e1] * sc;
+                if (a.qn) {
+                    x0 *= qn[e0];
+                    x1 *= qn[e1];
+                }
+                rope_rotate_fma(x0, x1, cr[p], sr[p]);
+                row[e0] = x0;
+                row[e1] = x1;
+                mx = fmaxf(mx, fmaxf(fabsf(x0), fabsf(x1)));
+            }
+        }
+        mx = group_max<LPR>(mx);
+        // 2^s with the largest element in [2^14, 2^15); 1 for zero and non-finite rows
+        const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
+        const int s = be == 0 || be == 255 ? 0 : min(141 - be, 126);
+        if (sub == 0) s_scale[wr][pr] = __uint_as_float((unsigned)(127 + s) << 23);
+    }
+    // ---- decode: the new row (the wave whose tiles end the range that ends the
+    // keys; each block of more than 16 heads writes the same bytes) ----
+    if constexpr (DECODE) {
+        if (owner) {
+            float* s_k = s_aux + AK;
+            if (a.kn) {
+                const float sc = rms_scale_ref_quad<HD>(s_k, lane & 3);
+                wave_sync();
+                for (int e = lane; e < HD; e += 64) s_k[e] = rms_apply(s_k[e], sc, s_aux[AKN + e]);
+                wave_sync();
+            }
+            const float* cr = s_aux + ACOS;
+            const float* sr = s_aux + ASIN;
+            const size_t off = (size_t)a.start * a.kv_dim + (size_t)kvh * HD;
+            for (int p = lane; p < HD / 2; p += 64) {
+                int e0, e1;
+                rope_pair(a.rope, p, HD, e0, e1);
+                float x0 = s_k[e0], x1 = s_k[e1];
+                rope_rotate(x0, x1, cr[p], sr[p]);
+                const uint16_t h0 = f32_to_f16_ref(x0), h1 = f32_to_f16_ref(x1);
+                s_new[0][e0] = h0;
+                s_new[0][e1] = h1;
+                a.kc[off + e0] = h0;
+                a.kc[off + e1] = h1;
+            }
+            for (int e = lane; e < HD; e += 64) {
+                const uint16_t h = f32_to_f16_ref(s_aux[AV + e]);
+                s_new[1][e] = h;
+                a.vc[off + e] = h;
+            }
+        }
+    }
+    if constexpr (KW > 1) __syncthreads();  // every wave's q rows
+    else wave_sync();
+
+    // q as the B operand: row c16, dims 32 ks + 8 g16 .. +7 (half step: 4 g16 .. +3)
+    half8 qh[KS], ql[KS];
+    half4 qh4 = {}, ql4 = {};
+    const float scl = s_scale[wr][c16];
+    const float sinv = __uint_as_float((254u << 23) - __float_as_uint(scl));  // 1 / scl
+    {
+        const float* row = qreg + c16 * QS;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float x = row[32 * ks + 8 * g16 + e] * scl;
+                qh[ks][e] = (_Float16)x;
+                ql[ks][e] = (_Float16)(x - (float)qh[ks][e]);
+            }
+        if constexpr (HALF) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float x = row[32 * KS + 4 * g16 + e] * scl;
+                qh4[e] = (_Float16)x;
+                ql4[e] = (_Float16)(x - (float)qh4[e]);
+            }
+        }
+    }
+
+    // operand addresses in a tile: K row c16 (+ 16), V rows 4 g16 + c16 / 4 (+ 16);
+    // the swizzle of row r + 16 is that of row r
+    int koff[KS], voff[DB];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) koff[ks] = c16 * T::ROWB + 16 * ((4 * ks + g16) ^ T::xk(c16));
+    const int koffh = c16 * T::ROWB + 16 * ((4 * KS + (g16 >> 1)) ^ T::xk(c16)) + 8 * (g16 & 1);
+    const int vr0 = 4 * g16 + (c16 >> 2);
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+        voff[db] = vr0 * T::ROWB + 16 * ((2 * db + ((c16 & 3) >> 1)) ^ T::xv(vr0)) + 8 * (c16 & 1);
+
+    const int qpos = a.start + min(R0 + c16, rlast) / a.g;             // of the lane's row
+    const int qmin = a.start + min(R0, rlast) / a.g;                   // of the wave's first row
+    const int qmax = R0 <= rlast ? a.start + min(R0 + kGmRows - 1, rlast) / a.g : -1;
+    float m_run = -1e30f, l_run = 0.0f;
+    floatx4 o[DB];  // O^T: dims 16 db + 4 g16 .. +3 of row c16
+#pragma unroll
+    for (int db = 0; db < DB; db++) o[db] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    auto compute = [&](int kt, int buf) __attribute__((always_inline)) {
+        const int key0 = kt * KEYS;
+        char* kl = lds[wk][buf][0];
+        char* vl = lds[wk][buf][1];
+        if constexpr (DECODE) {
+            if (owner && key0 + KEYS > a.start) {  // the last tile: the new row into its place
+                const int r = a.start - key0;
+                if (lane < T::CH) {
+                    *(u32x4*)(kl + r * T::ROWB + 16 * (lane ^ T::xk(r))) = ((const u32x4*)s_new[0])[lane];
+                    *(u32x4*)(vl + r * T::ROWB + 16 * (lane ^ T::xv(r))) = ((const u32x4*)s_new[1])[lane];
+                }
+                wave_sync();
+            }
+        }
+        floatx4 s[KB];
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++) s[kb] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            half8 kf[KB];
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) kf[kb] = *(const half8*)(kl + koff[ks] + kb * 16 * T::ROWB);
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[kb], qh[ks], s[kb], 0, 0, 0);
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[kb], ql[ks], s[kb], 0, 0, 0);
+        }
+        if constexpr (HALF) {
+            half4 kf[KB];
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) kf[kb] = *(const half4*)(kl + koffh + kb * 16 * T::ROWB);
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[kb], qh4, s[kb], 0, 0, 0);
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) s[kb] = __builtin_amdgcn_mfma_f32_16x16x16f16(kf[kb], ql4, s[kb], 0, 0, 0);
+        }
+        // keys key0 + 16 kb + 4 g16 + e of row c16
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[kb][e] *= sinv;
+        if (key0 + KEYS - 1 > qmin) {
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (key0 + 16 * kb + 4 * g16 + e > qpos) s[kb][e] = -__builtin_huge_valf();
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) mx = fmaxf(mx, s[kb][e]);
+        mx = max_x32(max_x16(mx));
+        if (__any(mx > m_run + kGmSlack)) {
+            const float m_new = fmaxf(m_run, mx);
+            const float corr = fast_exp2(m_run - m_new);
+            m_run = m_new;
+            l_run *= corr;
+#pragma unroll
+            for (int db = 0; db < DB; db++) o[db] *= corr;
+        }
+        const float mref = m_run - kGmShift;
+        // k-step h: keys 4 g16 .. +3 of key block 2 h, then of block 2 h + 1
+        half8 ph[KB / 2], pl[KB / 2];
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float p = fast_exp2(s[kb][e] - mref);
+                l_run += p;
+                const _Float16 hi = (_Float16)p;
+                ph[kb >> 1][4 * (kb & 1) + e] = hi;
+                pl[kb >> 1][4 * (kb & 1) + e] = (_Float16)(p - (float)hi);
+            }
+#pragma unroll
+        for (int h = 0; h < KB / 2; h++)
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                half4 part[2];
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    part[t] = __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) short4v*)(vl + voff[db] + (32 * h + 16 * t) * T::ROWB)));
+                const half8 vf = {part[0][0], part[0][1], part[0][2], part[0][3],
+                                  part[1][0], part[1][1], part[1][2], part[1][3]};
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[h], o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[h], o[db], 0, 0, 0);
+            }
+    };
+
+    int buf = 0;
+    for (int kt = tile0; kt < tile1; kt += KW) {
+        if constexpr (RW > 1) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's loads of the tile
+            __syncthreads();                                   // everyone's; the other buffer is free
+            issue(kt + 1, buf ^ 1);
+            if (kt * KEYS <= qmax) compute(kt, buf);
+        } else {
+            if (kt + KW < tile1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPW) : "memory");  // the next tile's stay in flight
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            compute(kt, buf);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the buffer has been read
+            issue(kt + 2 * KW, buf);
+        }
+        buf ^= 1;
+    }
+
+    // ---- the wave's result to LDS: rows of HD floats, the maximum and the sum ----
+    // (a prefill wave's over its own q rows, a decode wave's over its tiles)
+    float* res = DECODE ? (float*)&lds[wk][0][0][0] : qreg;
+    const float l = sum_x32(sum_x16(l_run));
+    float chk = l * 0.0f;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) chk = fmaf(o[db][e], 0.0f, chk);
+    const unsigned long long badl = __ballot(!(chk == 0.0f) && R0 + c16 <= rlast);
+    const unsigned bad = (unsigned)((badl | badl >> 16 | badl >> 32 | badl >> 48) & 0xFFFFu);
+    if (!((bad >> c16) & 1u)) {
+#pragma unroll
+        for (int db = 0; db < DB; db++) *(floatx4*)(res + c16 * QS + 16 * db + 4 * g16) = o[db];
+        if (g16 == 0) {
+            s_ml[w][0][c16] = m_run;
+            s_ml[w][1][c16] = l;
+        }
+    }
+    wave_sync();
+    if (bad) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the new row's stores
+        for (int r = 0; r < kGmRows; r++) {
+            if (!((bad >> r) & 1u)) continue;
+            float mr, lr;
+            gen_row<HD, KEYS>((const uint16_t*)kbase, (const uint16_t*)vbase, (size_t)a.kv_dim, qreg + r * QS,
+                        a.start + (R0 + r) / a.g, tile0, KW, tile1, lane, res + r * QS, mr, lr);
+            if (lane == 0) {
+                s_ml[w][0][r] = mr;
+                s_ml[w][1][r] = lr;
+            }
+        }
+        wave_sync();
+    }
+    if constexpr (KW > 1) __syncthreads();
+    const bool partial = a.nrange > 1;
+    const int nrow = min(kGmRows, rlast + 1 - R0);
+    for (int it = KW > 1 ? tid : lane; it < nrow * D4; it += KW > 1 ? 64 * NW : 64) {
+        const int r = it / D4, d4 = it - r * D4;
+        float M = -1e30f, L = 0.0f;
+        floatx4 A = {0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (KW == 1) {
+            M = s_ml[w][0][r];
+            L = s_ml[w][1][r];
+            A = *(const floatx4*)(res + r * QS + 4 * d4);
+        } else {
+#pragma unroll
+            for (int k = 0; k < KW; k++) M = fmaxf(M, s_ml[k][0][r]);
+#pragma unroll
+            for (int k = 0; k < KW; k++) {
+                const float e = fast_exp2(s_ml[k][0][r] - M);
+                L = fmaf(e, s_ml[k][1][r], L);
+                A += e * *(const floatx4*)((const float*)&lds[k][0][0][0] + r * QS + 4 * d4);
+            }
+        }
+        const int R = R0 + r;
+        const size_t orow = (size_t)(R / a.g) * a.nh + kvh * a.g + R % a.g;
+        if (partial) {
+            const size_t slot = (size_t)range * a.n_tok * a.nh + orow;
+            *(floatx4*)(a.part_acc + slot * HD + 4 * d4) = A;
+            if (d4 == 0) *(float2*)(a.part_ml + 2 * slot) = float2{M, L};
+        } else {
+            A *= 1.0f / L;
+            float* d = a.out + orow * HD + 4 * d4;
+            if (a.ovec) {
+                *(floatx4*)d = A;
+            } else {
+                *(float2*)d = float2{A[0], A[1]};
+                *(float2*)(d + 2) = float2{A[2], A[3]};
+            }
+        }
+    }
+}
+
+// out = sum_s 2^(m_s - M) acc_s / sum_s 2^(m_s - M) l_s over the ranges of one
+// output row: sg groups of hd / 4 threads per row, group j on ranges j, j + sg,
+// ..., summed through LDS. (An empty range has m = -1e30, weight 0.)
+constexpr int kGmMaxRanges = 256;
+__global__ __launch_bounds__(256) void gen_merge_kernel(const float* __restrict__ part_acc,
+                                                        const float* __restrict__ part_ml, float* __restrict__ out,
+                                                        int rows, int nrange, int hd, int sg, int ovec) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    const int d4n = hd >> 2, tpr = sg * d4n, rpw = 256 / tpr;
+    const int tid = threadIdx.x, rl = tid / tpr, j = (tid - rl * tpr) / d4n, d4 = tid - rl * tpr - j * d4n;
+    const int row = (int)blockIdx.x * rpw + rl;
+    const bool live = rl < rpw && row < rows;
+    float* s_m = sm;                                  // [rpw][nrange] maxima, then [rpw][nrange] sums
+    float* s_l = sm + rpw * nrange;
+    floatx4* s_a = (floatx4*)(sm + ((2 * rpw * nrange + 3) & ~3));  // [rpw][sg][d4n]
+    if (live)
+        for (int i = tid - rl * tpr; i < nrange; i += tpr) {
+            const float2 ml = *(const float2*)(part_ml + 2 * ((size_t)i * rows + row));
+            s_m[rl * nrange + i] = ml.x;
+            s_l[rl * nrange + i] = ml.y;
+        }
+    __syncthreads();
+    float M = -1e30f, L = 0.0f;
+    floatx4 A = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (live) {
+        for (int i = 0; i < nrange; i++) M = fmaxf(M, s_m[rl * nrange + i]);
+        for (int i = 0; i < nrange; i++) L = fmaf(fast_exp2(s_m[rl * nrange + i] - M), s_l[rl * nrange + i], L);
+#pragma unroll 8
+        for (int i = j; i < nrange; i += sg) {
+            const floatx4 v = *(const floatx4*)(part_acc + ((size_t)i * rows + row) * hd + 4 * d4);
+            A += fast_exp2(s_m[rl * nrange + i] - M) * v;
+        }
+        s_a[tid] = A;
+    }
+    __syncthreads();
+    if (live && j == 0) {
+        for (int k = 1; k < sg; k++) A += s_a[tid + k * d4n];
+        A *= 1.0f / L;
+        float* o = out + (size_t)row * hd + 4 * d4;
+        if (ovec) {
+            *(floatx4*)o = A;
+        } else {
+            *(float2*)o = float2{A[0], A[1]};
+            *(float2*)(o + 2) = float2{A[2], A[3]};
+        }
+    }
+}
+
+template <int HD>
+static void launch_gm(const GenMmaArgs& a, bool decode, unsigned grid, hipStream_t s) {
+    if (decode) hipLaunchKernelGGL((gen_mma_kernel<HD, true>), dim3(grid), dim3(64 * gm_decode_waves<HD>()), 0, s, a);
+    else hipLaunchKernelGGL((gen_mma_kernel<HD, false>), dim3(grid), dim3(256), 0, s, a);
+}
+
+hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, bool decode, const GenSrc& q, const GenSrc& k,
+                          const GenSrc& v, float* out, float* part_acc, float* part_ml, size_t part_rows) {
+    const int hd = ctx->head_dim;
+    const bool norm = ctx->has_qk_norm[layer] != 0;
+    GenMmaArgs a;
+    a.q = q;
+    a.k = k;
+    a.v = v;
+    a.qn = norm ? ctx->qk_norm + (size_t)layer * 2 * hd : nullptr;
+    a.kn = norm ? ctx->qk_norm + (size_t)layer * 2 * hd + hd : nullptr;
+    a.cos_tab = ctx->rope_cos;
+    a.sin_tab = ctx->rope_sin;
+    a.kc = ctx->key_cache + (size_t)layer * ctx->layer_elems;
+    a.vc = ctx->val_cache + (size_t)layer * ctx->layer_elems;
+    a.out = out;
+    a.part_acc = part_acc;
+    a.part_ml = part_ml;
+    a.start = start;
+    a.n_tok = n_tok;
+    a.nh = ctx->n_heads;
+    a.g = ctx->kv_mul;
+    a.n_kv = ctx->n_kv_heads;
+    a.kv_dim = (int)ctx->kv_dim;
+    a.rope = ctx->rope_style;
+    a.rows = n_tok * ctx->kv_mul;
+    const int rpb = decode ? kGmRows : 4 * kGmRows;
+    a.nblk = (a.rows + rpb - 1) / rpb;
+    a.qvec = ((uintptr_t)q.p & 15) == 0 && q.ld % 4 == 0;
+    a.ovec = ((uintptr_t)out & 15) == 0;
+    a.qscale = 1.4426950408889634f / sqrtf((float)hd);
+    // Ranges. Decode: about one workgroup per CU, each wave at least one 32-key tile; up
+    // to four tiles per wave need no second launch. Prefill: as long as the blocks
+    // leave CUs idle and a range keeps 512 keys (its q rows are prepared again).
+    const int tiles = (start + n_tok + 31) / 32;
+    const long long wgs = (long long)a.nblk * a.n_kv;
+    const int kw = decode ? (hd <= 128 ? 4 : 2) : 1;
+    long long ranges = std::max<long long>(1, (decode ? ctx->cu_count : 2LL * ctx->cu_count) / wgs);
+    ranges = std::min<long long>(ranges, decode ? (tiles <= 4 * kw ? 1 : (tiles + kw - 1) / kw) : std::max(1, tiles / 16));
+    ranges = std::min<long long>(ranges, kGmMaxRanges);
+    const size_t orows = (size_t)n_tok * a.nh;
+    ranges = std::max<long long>(1, std::min<long long>(ranges, (long long)(part_rows / orows)));
+    a.nrange = (int)ranges;
+    const long long grid = wgs * ranges;
+    if (grid > 0x7FFFFFFF || orows > 0x7FFFFFFF) return hipErrorInvalidValue;
+    switch (hd) {
+#define PQA_GM(H) case H: launch_gm<H>(a, decode, (unsigned)grid, ctx->stream); break;
+        PQA_GM(80) PQA_GM(96) PQA_GM(112) PQA_GM(160) PQA_GM(192) PQA_GM(256)
+#undef PQA_GM
+        default: return hipErrorInvalidValue;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || ranges == 1) return e;
+    const int sg = std::min<int>((int)ranges, 256 / (hd / 4)), rpw = 256 / (sg * (hd / 4));
+    const size_t lds = ((2 * (size_t)rpw * ranges + 3) & ~(size_t)3) * 4 + 256 * 16;
+    hipLaunchKernelGGL(gen_merge_kernel, dim3((unsigned)((orows + rpw - 1) / rpw)), dim3(256), lds, ctx->stream,
+                       (const float*)part_acc, (const float*)part_ml, out, (int)orows, (int)ranges, hd, sg, a.ovec);
+    return hipGetLastError();
+}
+
+}  // namespace pqa

@@ -103,7 +103,7 @@ struct pqa_ctx {
     float* battn = nullptr;  // pqa_prefill_block's attention rows [n_tok][q_dim]
     size_t battn_floats = 0;
 
-    // head sizes other than 64 and 128 (pqa_general.hip): the prepared q rows,
+    // head sizes on the VALU kernels of pqa_general.hip: the prepared q rows,
     // one token's worth from context creation on, grown by prompts
     float* gen_q = nullptr;
     size_t gen_q_floats = 0;
@@ -135,8 +135,12 @@ struct pqa_ctx {
 
 namespace pqa {
 
-// head sizes with MFMA kernels; other even sizes up to 512 take pqa_general.hip
+// head sizes with MFMA kernels of their own; other even sizes up to 512 take the
+// general path, on the matrix cores for the sizes models use (pqa_general_mma.hip)
 inline bool mfma_head_dim(int hd) { return hd == 64 || hd == 128; }
+inline bool gen_mma_head_dim(int hd) {
+    return hd == 80 || hd == 96 || hd == 112 || hd == 160 || hd == 192 || hd == 256;
+}
 constexpr int kMaxHeadDim = 512;
 
 int set_err(pqa_ctx* ctx, int code, const std::string& msg);

@@ -114,3 +114,96 @@ def test_prefill_key_ranges(nh, nkv, hd, start, n_tok, split_q):
         mag = O.attend_f64(shp, start + t, qr[t], kc, vc & 0x7FFF)
         assert np.all(np.abs(out[t] - want) <= rel * mag + 1e-6), t
     att.close()
+
+
+# the matrix-core kernels of the other head sizes: history lengths around their 32-key tiles, one
+# and several tiles per wave, one and several key ranges (decode and prefill), GQA groups of 1 to
+# 20 heads (more than 16: two row blocks), every size and RoPE pairing
+GEN = [(80, 4, 4, 0), (96, 8, 2, 31), (112, 7, 1, 32), (160, 20, 1, 33), (192, 6, 2, 127), (256, 8, 1, 128),
+       (80, 17, 1, 513), (96, 32, 8, 3001), (256, 16, 2, 2500), (160, 3, 3, 1100), (112, 12, 4, 4100), (192, 2, 1, 700)]
+
+
+def _gen_case(hd, nh, nkv, start, n_tok, style, seed):
+    smax, kvd = start + n_tok, nkv * hd
+    cos, sin = O.rope_table(1e6, hd, smax)
+    att = PicoAttention(1, smax, nh, nkv, hd, style, rope_cos=cos, rope_sin=sin)
+    qn, kn = O.qk_norm_weights(seed, 0, hd)
+    att.set_qk_norm(0, qn, kn)
+    att.synth_kv(0, 0, start, seed, 0.01)
+    kc, vc = np.zeros((smax, kvd), np.uint16), np.zeros((smax, kvd), np.uint16)
+    kc[:start], vc[:start] = O.synth_kv_rows(seed, 0, kvd, 0, start, 0.01)
+    q, k, v = O.batch_inputs(seed, 0, 0, n_tok, nh, nkv, hd)
+    return att, q, k, v, qn, kn, cos, sin, kc, vc
+
+
+def _check_gen(att, shp, start, toks, out, q, k, v, qn, kn, cos, sin, kc, vc):
+    qr = [O.append(shp, start + t, q[t], k[t], v[t], qn, kn, cos[start + t], sin[start + t], kc, vc)
+          for t in range(q.shape[0])]
+    gk, gv = att.kv_download(0, start, q.shape[0])
+    assert_bits_equal(gk, kc[start:], "K rows")
+    assert_bits_equal(gv, vc[start:], "V rows")
+    for t in toks:
+        want = O.attend_f64(shp, start + t, qr[t], kc, vc)
+        mag = O.attend_f64(shp, start + t, qr[t], kc, vc & 0x7FFF)
+        # 22-bit operands and fp32 sums: a score is off by at most 2^-20 sum |q k| log2(e) / sqrt(hd), with the x8
+        # outlier rows below 2^-20 * 150; twice that, times ln 2, relative to sum p |v|
+        assert np.all(np.abs(out[t] - want) <= 2.0 ** -12 * mag), t
+        # and in the mean square far below it
+        assert np.sqrt(np.mean((out[t] - want) ** 2)) <= 2.0 ** -18 * np.sqrt(np.mean(mag ** 2)), t
+
+
+@pytest.mark.parametrize("hd,nh,nkv,pos", GEN)
+def test_general_mma_decode(hd, nh, nkv, pos):
+    style, seed = (hd // 16) % 3, 5100 + pos
+    print(f"general decode {nh}/{nkv} x {hd} at {pos}, rope {style}", flush=True)
+    att, q, k, v, qn, kn, cos, sin, kc, vc = _gen_case(hd, nh, nkv, pos, 1, style, seed)
+    out = att.forward(0, pos, *(torch.from_numpy(x[0]).to(DEV) for x in (q, k, v))).cpu().numpy()
+    _check_gen(att, O.shape(nh, nkv, hd, pos + 1, style), pos, [0], out[None], q, k, v, qn, kn, cos, sin, kc, vc)
+    att.close()
+
+
+@pytest.mark.parametrize("n_tok", [1, 17, 70])
+@pytest.mark.parametrize("hd,nh,nkv,start", GEN)
+def test_general_mma_prefill(hd, nh, nkv, start, n_tok):
+    style, seed = (hd // 16 + 1) % 3, 5200 + start
+    print(f"general prefill {nh}/{nkv} x {hd}, {n_tok} tokens at {start}, rope {style}", flush=True)
+    att, q, k, v, qn, kn, cos, sin, kc, vc = _gen_case(hd, nh, nkv, start, n_tok, style, seed)
+    flat = torch.empty(n_tok * nh * hd + 2, device=DEV)
+    o = flat[2:].view(n_tok, nh * hd)  # 8-byte aligned output, 4-byte aligned q
+    qd = torch.empty(q.size + 1, device=DEV)[1:].view(q.shape)
+    qd.copy_(torch.from_numpy(q))
+    att.forward_batch(0, start, qd, torch.from_numpy(k).to(DEV), torch.from_numpy(v).to(DEV), out=o)
+    out = o.cpu().numpy()
+    _check_gen(att, O.shape(nh, nkv, hd, start + n_tok, style), start, sorted({0, n_tok // 2, n_tok - 1}), out, q, k, v,
+               qn, kn, cos, sin, kc, vc)
+    att.close()
+
+
+@pytest.mark.parametrize("hd", [80, 96, 256])
+def test_general_mma_non_finite_rows(hd):
+    # rows that overflow fp16 (infinities in the cache): tokens before them are untouched, a key of score -inf
+    # has weight 0, and what is infinite or NaN in the reference's arithmetic stays so
+    print(f"general path, infinite cache rows, hd {hd}", flush=True)
+    nh, nkv, n_tok, seed = 4, 1, 45, 5300 + hd
+    cos, sin = np.ones((n_tok, hd // 2), np.float32), np.zeros((n_tok, hd // 2), np.float32)  # no rotation
+    att = PicoAttention(1, n_tok, nh, nkv, hd, 0, rope_cos=cos, rope_sin=sin)
+    q, k, v = (x.copy() for x in O.batch_inputs(seed, 0, 0, n_tok, nh, nkv, hd))
+    q[:, 0::hd] = np.abs(q[:, 0::hd]) + 0.1   # dim 0 of every head: positive, and
+    k[20, 0] = -1e6                           # row 20's score -inf
+    v[33, 5] = 1e6                            # dim 5 infinite from token 33 on
+    v[40, 7] = np.nan
+    out = att.forward_batch(0, 0, *(torch.from_numpy(x).to(DEV) for x in (q, k, v))).cpu().numpy()
+    shp = O.shape(nh, nkv, hd, n_tok, 0)
+    kc, vc = np.zeros((n_tok, nkv * hd), np.uint16), np.zeros((n_tok, nkv * hd), np.uint16)
+    for t in range(n_tok):
+        qr = O.append(shp, t, q[t], k[t], v[t], None, None, cos[t], sin[t], kc, vc)
+        want = O.attend(shp, t, qr, kc, vc)
+        assert np.array_equal(np.isnan(out[t]), np.isnan(want)), t
+        assert np.array_equal(np.isinf(out[t]), np.isinf(want)), t
+        fin = np.isfinite(want)
+        assert np.all(np.abs(out[t][fin] - want[fin]) <= 1e-4), t
+    # the same through the decode: the last token again, over the rows just written
+    t = n_tok - 1
+    dec = att.forward(0, t, *(torch.from_numpy(x[t]).to(DEV) for x in (q, k, v))).cpu().numpy()
+    assert np.array_equal(np.isnan(dec), np.isnan(want)) and np.array_equal(np.isinf(dec), np.isinf(want))
+    att.close()
