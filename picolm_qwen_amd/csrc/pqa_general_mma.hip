@@ -27,10 +27,10 @@
 //
 // Measured per layer against the VALU kernels (launch count, all kernels): decode of
 // 32 / 8 heads of 96 at 9000 44 -> 22 us (13 us for the 27.6 MB of cache, merge 4;
-// the rest is the gap between two launches), 8 / 2 heads of 256 at 4 16 -> 6 us;
+// the rest is the gap between two launches), 8 / 2 heads of 256 at 4 37 -> 15 us;
 // prefill of 700 tokens at head size 96 226 -> 41 us (kernel 207 -> 25; its bound is
-// the chain of one tile: operand reads, products, softmax, products), 851 at 256
-// 248 -> 46. The error against 64-bit sums is 0.6 to 0.8 times theirs.
+// the chain of one tile: operand reads, products, softmax, products), 851 tokens at
+// 256 353 -> 71. The error of a decode against 64-bit sums is 0.25 to 0.8 times theirs.
 //
 // Infinities: a split product can turn inf into NaN (inf * 0, inf - inf), and a
 // masked key's V row still enters the product with weight 0. A row whose result is
