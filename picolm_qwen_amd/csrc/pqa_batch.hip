@@ -25,6 +25,7 @@
 
 #include "pqa_device.h"
 #include "pqa_internal.h"
+#include "pqa_ordered.h"
 
 namespace pqa {
 
@@ -131,11 +132,9 @@ __global__ __launch_bounds__(256) void split2_kernel(const float* __restrict__ s
 // aligned: the row is read once into registers as float4s and written as
 // half4s (same arithmetic, same bits).
 constexpr int kSplitVec = 8;
-__global__ __launch_bounds__(256) void split2_vec_kernel(const float* __restrict__ src, int n,
-                                                         _Float16* __restrict__ dst, int kh,
-                                                         float* __restrict__ inv_scale) {
-    __shared__ float s_max[4];
-    const int row = blockIdx.x, tid = threadIdx.x;
+__device__ __forceinline__ void split2_vec_row(const float* __restrict__ src, int n, _Float16* __restrict__ dst, int kh,
+                                               float* __restrict__ inv_scale, int row, float* s_max) {
+    const int tid = threadIdx.x;
     const int n4 = n >> 2;
     const float4* a = (const float4*)(src + (size_t)row * n);
     _Float16* d = dst + (size_t)row * 2 * kh;
@@ -171,14 +170,58 @@ __global__ __launch_bounds__(256) void split2_vec_kernel(const float* __restrict
     }
 }
 
+__global__ __launch_bounds__(256) void split2_vec_kernel(const float* __restrict__ src, int n,
+                                                         _Float16* __restrict__ dst, int kh,
+                                                         float* __restrict__ inv_scale) {
+    __shared__ float s_max[4];
+    split2_vec_row(src, n, dst, kh, inv_scale, blockIdx.x, s_max);
+}
+
+// The inputs split and, in the workgroups past the rows, their image for the
+// reference-order projection: one launch for the two readers of X (a launch of
+// its own costs a short prompt 5 us).
+template <bool Q8>
+__global__ __launch_bounds__(256) void split2_image_kernel(const float* __restrict__ src, int n,
+                                                           _Float16* __restrict__ dst, int kh,
+                                                           float* __restrict__ inv_scale, int rows,
+                                                           float* __restrict__ image) {
+    __shared__ float s_max[4];
+    __shared__ __attribute__((aligned(16))) float img[4 * kOrdStageF];
+    if ((int)blockIdx.x < rows) {
+        split2_vec_row(src, n, dst, kh, inv_scale, blockIdx.x, s_max);
+    } else {
+        const int groups = (ord_stages(Q8, n) + 3) / 4, i = (int)blockIdx.x - rows;
+        ordered_image_tile<Q8>(src, n, rows, n, image, i % groups, i / groups, img);
+    }
+}
+
+static bool split_vec(const float* src, int n) {
+    return n % 4 == 0 && n <= 256 * 4 * kSplitVec && ((uintptr_t)src & 15) == 0;
+}
+
 // one workgroup per row of src [rows][n] into dst [rows][2 kh], kh = k_half(n)
 static void launch_split2(const float* src, int rows, int n, _Float16* dst, int kh, float* inv_scale,
                           hipStream_t stream) {
-    const bool vec = n % 4 == 0 && n <= 256 * 4 * kSplitVec && ((uintptr_t)src & 15) == 0;
-    if (vec)
+    if (split_vec(src, n))
         hipLaunchKernelGGL(split2_vec_kernel, dim3(rows), dim3(256), 0, stream, src, n, dst, kh, inv_scale);
     else
         hipLaunchKernelGGL(split2_kernel, dim3(rows), dim3(256), 0, stream, src, n, dst, kh, inv_scale);
+}
+
+// The same with the rows' image (q8: in the Q8_0 order).
+static hipError_t launch_split2_image(const float* src, int rows, int n, _Float16* dst, int kh, float* inv_scale,
+                                      bool q8, float* image, hipStream_t stream) {
+    if (!split_vec(src, n)) {
+        launch_split2(src, rows, n, dst, kh, inv_scale, stream);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : launch_ordered_image(q8, src, n, rows, n, image, stream);
+    }
+    const dim3 grid(rows + (ord_stages(q8, n) + 3) / 4 * ((rows + kOrdTile - 1) / kOrdTile));
+    if (q8)
+        hipLaunchKernelGGL(split2_image_kernel<true>, grid, dim3(256), 0, stream, src, n, dst, kh, inv_scale, rows, image);
+    else
+        hipLaunchKernelGGL(split2_image_kernel<false>, grid, dim3(256), 0, stream, src, n, dst, kh, inv_scale, rows, image);
+    return hipGetLastError();
 }
 
 // each half of a split row: n rounded up to the GEMM's 32-wide k tiles
@@ -251,22 +294,11 @@ __global__ __launch_bounds__(256) void unscale_residual_kernel(const float* __re
     *xp = o;
 }
 
-// y[t][c] = the sum of the GEMM's K slices part[s][t][c] in slice order, c < cols
-// (an even number) of y's ld columns. Thread: 2 columns of one token.
-__global__ __launch_bounds__(256) void sum_slices_kernel(const float* __restrict__ part, int slices,
-                                                         size_t slice_stride, int cols, float* __restrict__ y, int ld) {
-    const int t = blockIdx.y;
-    const int c = 2 * (blockIdx.x * 256 + threadIdx.x);
-    if (c >= cols) return;
-    const float* p = part + (size_t)t * cols + c;
-    float2 v = *(const float2*)p;
-#pragma unroll 4
-    for (int s = 1; s < slices; s++) {
-        const float2 u = *(const float2*)(p + s * slice_stride);
-        v.x = v.x + u.x;
-        v.y = v.y + u.y;
-    }
-    *(float2*)(y + (size_t)t * ld + c) = v;
+__global__ __launch_bounds__(256) void sum_slices_kernel(const SliceSum a) { sum_slices(a, blockIdx.x); }
+
+hipError_t launch_sum_slices(const SliceSum& a, hipStream_t s) {
+    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)sum_slices_blocks(a)), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_dequant_rows(int type, const void* w, int stride, int rows, int n, float* dst, hipStream_t s) {
@@ -402,8 +434,8 @@ static size_t image_floats(const pqa_proj_weights& p, int n_tok) {
 }
 
 // k[t * ldo + r] and v[t * ldo + r] = the attn_k / attn_v matmul_bias of token
-// t in the reference's order (pqa_exact.hip), bit-exact. image: image_floats of
-// workspace.
+// t in the reference's order (pqa_exact.hip), bit-exact. image: attn_k's image of
+// the inputs (batch_gemm makes it), in image_floats of workspace.
 static int exact_kv(pqa_ctx* ctx, int layer, int n_tok, const float* xb, float* image, float* k, float* v, int ldo,
                     const char* fn) {
     if (int rc = ensure_layer_exact(ctx, layer, fn)) return rc;
@@ -413,12 +445,10 @@ static int exact_kv(pqa_ctx* ctx, int layer, int n_tok, const float* xb, float* 
     const float* wv = p.exact + pqa::exact_matrix_floats(p.wtype[1], rows, n);
     const pqa::OrderedProj kv[2] = {{p.wtype[1], wk, p.b[1], p.btype[1], k}, {p.wtype[2], wv, p.b[2], p.btype[2], v}};
     const bool qk = p.wtype[1] == pqa::GG_Q8_0, qv = p.wtype[2] == pqa::GG_Q8_0;
-    hipError_t e = pqa::launch_ordered_image(qk, xb, n, n_tok, n, image, ctx->stream);
-    if (e == hipSuccess)
-        e = pqa::launch_ordered_project(kv, qk == qv ? 2 : 1, rows, n, image, n_tok, ldo, ctx->stream);
+    hipError_t e = pqa::launch_ordered_project(kv, qk == qv ? 2 : 1, rows, n, image, n_tok, ldo, ctx->cu_count, ctx->stream);
     if (e == hipSuccess && qk != qv) {
         e = pqa::launch_ordered_image(qv, xb, n, n_tok, n, image, ctx->stream);
-        if (e == hipSuccess) e = pqa::launch_ordered_project(kv + 1, 1, rows, n, image, n_tok, ldo, ctx->stream);
+        if (e == hipSuccess) e = pqa::launch_ordered_project(kv + 1, 1, rows, n, image, n_tok, ldo, ctx->cu_count, ctx->stream);
     }
     return hip_check(ctx, e, fn);
 }
@@ -495,8 +525,10 @@ static BatchShape out_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n
 // element scaled by 2^(s_w[c] + s_x[t]); *w_inv = the inverse column scales.
 // q_only: the GEMM covers the q columns alone (the reference-order projection
 // fills the k and v columns).
+// K slices of the GEMM are left to the caller: *sum says what makes sb->y of them
+// (0 slices: nothing).
 static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, SplitBufs* sb, const float** w_inv,
-                      const char* fn, bool q_only = false) {
+                      pqa::SliceSum* sum, const char* fn, bool q_only) {
     const int n = ctx->proj[layer].n_embd;
     if (int rc = ensure_layer_split(ctx, layer, fn)) return rc;
     const auto& p = ctx->proj[layer];
@@ -506,8 +538,14 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
     *w_inv = (const float*)((const char*)p.split + up256(total * 2 * kh * 2));
     const BatchShape bs = qkv_shape(ctx, p, n_tok, q_only);
     if (int rc = ensure_split(ctx, n_tok, n, bs.y_floats, bs.part_floats, bs.image, sb, fn)) return rc;
-    pqa::launch_split2(xb, n_tok, n, sb->x3, kh, sb->x_inv, ctx->stream);
-    if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
+    if (q_only) {
+        const hipError_t e = pqa::launch_split2_image(xb, n_tok, n, sb->x3, kh, sb->x_inv, p.wtype[1] == pqa::GG_Q8_0,
+                                                      sb->image, ctx->stream);
+        if (int rc = hip_check(ctx, e, fn)) return rc;
+    } else {
+        pqa::launch_split2(xb, n_tok, n, sb->x3, kh, sb->x_inv, ctx->stream);
+        if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
+    }
     // Y[n_tok][total] = X_hi W_hi^T + X_hi W_lo^T + X_lo W_hi^T (the q rows come first)
     const int cols = q_only ? (int)ctx->q_dim : (int)total;
     const bool sliced = bs.plan.slices > 1;
@@ -516,10 +554,8 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
         pqa::launch_gemm_f16x3_nt(bs.plan, sb->x3, 2 * kh, w3, 2 * kh, sliced ? sb->parts : sb->y,
                                   sliced ? cols : (int)total, stride, n_tok, cols, kh, ctx->stream);
     if (int rc = hip_check(ctx, e, fn)) return rc;
-    if (sliced)
-        hipLaunchKernelGGL(pqa::sum_slices_kernel, dim3((cols / 2 + 255) / 256, n_tok), dim3(256), 0, ctx->stream,
-                           (const float*)sb->parts, bs.plan.slices, stride, cols, sb->y, (int)total);
-    return hip_check(ctx, hipGetLastError(), fn);
+    *sum = pqa::SliceSum{sb->parts, sb->y, stride, sliced ? bs.plan.slices : 0, cols, (int)total, n_tok};
+    return PQA_OK;
 }
 
 static int check_batch(pqa_ctx* ctx, int layer, int n_tok, const char* fn) {
@@ -547,7 +583,10 @@ extern "C" int pqa_qkv_project_batch(pqa_ctx* ctx, int layer, int n_tok, const f
         if (int rc = ensure_layer_exact(ctx, layer, fn)) return rc;
     SplitBufs sb;
     const float* w_inv = nullptr;
-    if (int rc = batch_gemm(ctx, layer, n_tok, xb, &sb, &w_inv, fn, exact)) return rc;
+    pqa::SliceSum sum;
+    if (int rc = batch_gemm(ctx, layer, n_tok, xb, &sb, &w_inv, &sum, fn, exact)) return rc;
+    if (sum.slices)
+        if (int rc = hip_check(ctx, pqa::launch_sum_slices(sum, ctx->stream), fn)) return rc;
     const auto& p = ctx->proj[layer];
     const size_t total = ctx->q_dim + 2 * ctx->kv_dim;
     pqa::ScatterArgs sa;
@@ -582,7 +621,8 @@ extern "C" int pqa_prefill_x(pqa_ctx* ctx, int layer, int start_pos, int n_tok, 
         if (int rc = ensure_layer_exact(ctx, layer, fn)) return rc;
     SplitBufs sb;
     const float* w_inv = nullptr;
-    if (int rc = batch_gemm(ctx, layer, n_tok, xb, &sb, &w_inv, fn, exact)) return rc;
+    pqa::SliceSum sum;
+    if (int rc = batch_gemm(ctx, layer, n_tok, xb, &sb, &w_inv, &sum, fn, exact)) return rc;
     const auto& p = ctx->proj[layer];
     const int ld = (int)(ctx->q_dim + 2 * ctx->kv_dim);
     if (exact)  // the k and v columns of the GEMM result, in the reference's order
@@ -598,6 +638,11 @@ extern "C" int pqa_prefill_x(pqa_ctx* ctx, int layer, int start_pos, int n_tok, 
         ys.bt[i] = p.btype[i];
     }
     ys.kv_plain = exact;
+    ys.sum = sum;
+    if (sum.slices && !exact) {  // the K/V prep reads the summed k and v columns
+        if (int rc = hip_check(ctx, pqa::launch_sum_slices(sum, ctx->stream), fn)) return rc;
+        ys.sum.slices = 0;
+    }
     return hip_check(ctx, pqa::launch_prefill_scaled(ctx, layer, start_pos, n_tok, ys, out), fn);
 }
 

@@ -165,6 +165,24 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// 256 threads of workgroup `block` of sum_slices_blocks: 2 columns each (S: SliceSum)
+template <class S>
+__device__ __forceinline__ void sum_slices(const S& a, int block) {
+    const int half = a.cols >> 1;
+    const long long i = (long long)block * 256 + threadIdx.x;
+    if (i >= (long long)a.n_tok * half) return;
+    const int t = (int)(i / half), c = 2 * (int)(i - (long long)t * half);
+    const float* p = a.part + (size_t)t * a.cols + c;
+    float2 v = *(const float2*)p;
+#pragma unroll 4
+    for (int s = 1; s < a.slices; s++) {
+        const float2 u = *(const float2*)(p + s * a.stride);
+        v.x = v.x + u.x;
+        v.y = v.y + u.y;
+    }
+    *(float2*)(a.y + (size_t)t * a.ld + c) = v;
+}
+
 // A pointer the caller knows to be wave-uniform, moved to scalar registers.
 __device__ __forceinline__ const void* uniform_ptr(const void* p) {
     const unsigned long long v = (unsigned long long)p;

@@ -50,33 +50,13 @@
 
 #include "pqa_device.h"
 #include "pqa_internal.h"
+#include "pqa_ordered.h"
 
 namespace pqa {
 
 typedef float floatx32 __attribute__((ext_vector_type(32)));
 
-constexpr int kOrdTile = 32;                      // tokens and rows per workgroup
-constexpr int kOrdK = 64;                         // k elements per stage: 8 of each of the 8 sequences
 constexpr int kOrdThreads = 256;                  // 4 waves
-constexpr int kOrdStageF = kOrdTile * kOrdK;      // floats of one operand's stage
-
-__host__ __device__ inline int ord_stages(bool q8, int n) { return q8 ? (n + 255) / 256 * 4 : (n + kOrdK - 1) / kOrdK; }
-
-// element k of a row: its stage, and its float within the stage's image at lane row `r`
-__device__ __forceinline__ void ord_place(bool q8, int k, int r, int& st, int& f) {
-    int c, j;  // sequence and element of the stage
-    if (q8) {
-        st = (k >> 8) * 4 + ((k >> 3) & 3);
-        c = (k >> 5) & 7;
-        j = k & 7;
-    } else {
-        st = k >> 6;
-        c = k & 7;
-        j = (k >> 3) & 7;
-    }
-    const int q = q8 ? c >> 1 : c & 3, b = q8 ? c & 1 : c >> 2;
-    f = (2 * q + (j >> 2)) * 256 + (32 * b + r) * 4 + (j & 3);
-}
 
 struct OrderedArgs {
     const float* w[2];  // images of the weight rows (Q8_0: the int8 values as floats)
@@ -93,50 +73,75 @@ __device__ __forceinline__ float ord_bias(const uint8_t* b, int bt, int r) {
     return bt == GG_F32 ? ((const float*)b)[r] : f16_bits_to_f32(((const uint16_t*)b)[r]);
 }
 
-template <bool Q8>
+// S: tokens and rows per MFMA tile. 32: the workgroup is one tile, a wave takes
+// two sequences (v_mfma_f32_32x32x1_2b). 16: two tiles of 16 tokens x 16 rows, two
+// waves each, a wave takes four (v_mfma_f32_16x16x1_4b), for prompts whose 32 x 32
+// tiles would leave SIMDs idle or with a lone wave.
+template <int S> struct OrdMfma;
+template <> struct OrdMfma<32> {
+    typedef floatx32 Acc;
+    __device__ static Acc mul(float a, float b, Acc z) { return __builtin_amdgcn_mfma_f32_32x32x1f32(a, b, z, 0, 0, 0); }
+};
+template <> struct OrdMfma<16> {
+    typedef floatx16 Acc;
+    __device__ static Acc mul(float a, float b, Acc z) { return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, z, 0, 0, 0); }
+};
+
+template <bool Q8, int S>
 __global__ __launch_bounds__(kOrdThreads, 4) void ordered_kernel(const OrderedArgs a) {
 #pragma clang fp contract(off)
     constexpr int PD = Q8 ? 2 : 3;  // stages in registers (Q8_0: a third does not fit four waves per SIMD)
-    constexpr int NR = 16;  // results per lane of the whole tile
-    __shared__ float ex[Q8 ? 8 * NR * 64 : 4 * NR * 64];  // [block or wave][result][lane]
+    constexpr int NB = 64 / S;                 // sequences per wave = MFMA blocks
+    constexpr int NR = S * S / 64;             // results per lane of a whole tile
+    constexpr int WT = 8 / NB;                 // waves per tile
+    constexpr int NF = NR / WT;                // results a wave finishes
+    constexpr int NX = Q8 ? 8 : S == 32 ? 4 : 2;  // exchanged values per result: blocks, or waves
+    __shared__ float ex[4 / WT][NX * NR * 64];    // [tile][block or wave][result][lane]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int q = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hb = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = w % WT, half = w / WT;          // wave of its tile; the tile's rows 16 half .. +15
+    const int li = lane % S, blk_l = lane / S;    // token / row and MFMA block of the lane's operands
     const int mat = (int)blockIdx.x >= a.rtiles ? 1 : 0;
     const int rt = (int)blockIdx.x - mat * a.rtiles;
-    const int r0 = rt * kOrdTile, t0 = (int)blockIdx.y * kOrdTile;
+    const int r0 = rt * kOrdTile + half * S, t0 = (int)blockIdx.y * S;
     const int nst = ord_stages(Q8, a.n);
-    const float* xt = a.x + ((size_t)blockIdx.y * nst * kOrdStageF + 512 * q);
-    const float* wt = a.w[mat] + ((size_t)rt * nst * kOrdStageF + 512 * q);
+    // the lane's sequence; chain types so that the chains l and l + 4 (and, with
+    // four blocks, l + 2 and l + 6) of the final sum meet in one lane
+    const int seq = Q8 ? NB * q + blk_l : S == 32 ? q + 4 * blk_l : q + (blk_l & 1) * 4 + (blk_l >> 1) * 2;
+    int st_unused, f_x, f_w;  // the lane's 16 bytes of a stage (half 0)
+    ord_place(Q8, Q8 ? 32 * seq : seq, t0 % kOrdTile + li, st_unused, f_x);
+    ord_place(Q8, Q8 ? 32 * seq : seq, half * S + li, st_unused, f_w);
+    const float* xt = a.x + (size_t)(t0 / kOrdTile) * nst * kOrdStageF + f_x;
+    const float* wt = a.w[mat] + (size_t)rt * nst * kOrdStageF + f_w;
 
     floatx4 xv[PD][2], wv[PD][2];
     auto load = [&](int st, int p) __attribute__((always_inline)) {
         const size_t o = (size_t)min(st, nst - 1) * kOrdStageF;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            xv[p][h] = *(const floatx4*)(xt + o + 256 * h + 4 * lane);
-            wv[p][h] = *(const floatx4*)(wt + o + 256 * h + 4 * lane);
+            xv[p][h] = *(const floatx4*)(xt + o + 256 * h);
+            wv[p][h] = *(const floatx4*)(wt + o + 256 * h);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    floatx32 acc;  // sums of this wave's two sequences: MFMA result layout, block b at 16 b
-    floatx32 zero;
+    typename OrdMfma<S>::Acc acc;  // sums of this wave's sequences: MFMA result layout, block b at NR b
+    typename OrdMfma<S>::Acc zero;
 #pragma unroll
-    for (int e = 0; e < 32; e++) acc[e] = zero[e] = 0.0f;
-    float sumf[Q8 ? 4 : 1];  // Q8_0: results 4 q .. +3
+    for (int e = 0; e < NB * NR; e++) acc[e] = zero[e] = 0.0f;
+    float sumf[Q8 ? NF : 1];  // Q8_0: results NF q ..
 #pragma unroll
-    for (int e = 0; e < (Q8 ? 4 : 1); e++) sumf[e] = 0.0f;
+    for (int e = 0; e < (Q8 ? NF : 1); e++) sumf[e] = 0.0f;
 
     auto compute = [&](int p) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             float x = xv[p][u >> 2][u & 3];
             asm volatile("" : "+v"(x));  // keeps this MFMA behind the sums before it: one product buffer
-            const floatx32 pr = __builtin_amdgcn_mfma_f32_32x32x1f32(x, wv[p][u >> 2][u & 3], zero, 0, 0, 0);
+            const typename OrdMfma<S>::Acc pr = OrdMfma<S>::mul(x, wv[p][u >> 2][u & 3], zero);
 #pragma unroll
-            for (int e = 0; e < 32; e++) acc[e] = acc[e] + pr[e];
+            for (int e = 0; e < NB * NR; e++) acc[e] = acc[e] + pr[e];
             asm volatile("" : "+v"(acc));
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -147,31 +152,31 @@ __global__ __launch_bounds__(kOrdThreads, 4) void ordered_kernel(const OrderedAr
     auto step = [&](int st, int p) __attribute__((always_inline)) {
         compute(p);
         load(st + PD, p);
-                    if constexpr (Q8) {
-                        if ((st & 3) == 3) {
-                            // the round's 8 blocks: d * sum of each, then added in block order
-                            const int blk0 = 2 * (st & ~3), nblk = a.n / 32;
-                            const float* dr = a.d[mat] + (size_t)min(r0 + l32, a.rows - 1) * nblk;
-                            float d[2];
-        #pragma unroll
-                            for (int b = 0; b < 2; b++) d[b] = dr[min(blk0 + 2 * q + b, nblk - 1)];
-                            __syncthreads();  // the last round has been read
-        #pragma unroll
-                            for (int b = 0; b < 2; b++)
-        #pragma unroll
-                                for (int e = 0; e < 16; e++) ex[((2 * q + b) * NR + e) * 64 + lane] = d[b] * acc[16 * b + e];
-                            __syncthreads();
-        #pragma unroll
-                            for (int b = 0; b < 8; b++) {
-                                if (blk0 + b < nblk) {
-        #pragma unroll
-                                    for (int e = 0; e < 4; e++) sumf[e] = sumf[e] + ex[(b * NR + 4 * q + e) * 64 + lane];
-                                }
-                            }
-        #pragma unroll
-                            for (int e = 0; e < 32; e++) acc[e] = 0.0f;
-                        }
+        if constexpr (Q8) {
+            if ((st & 3) == 3) {
+                // the round's 8 blocks: d * sum of each, then added in block order
+                const int blk0 = 2 * (st & ~3), nblk = a.n / 32;
+                const float* dr = a.d[mat] + (size_t)min(r0 + li, a.rows - 1) * nblk;
+                float d[NB];
+#pragma unroll
+                for (int b = 0; b < NB; b++) d[b] = dr[min(blk0 + NB * q + b, nblk - 1)];
+                __syncthreads();  // the last round has been read
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int e = 0; e < NR; e++) ex[half][((NB * q + b) * NR + e) * 64 + lane] = d[b] * acc[NR * b + e];
+                __syncthreads();
+#pragma unroll
+                for (int b = 0; b < 8; b++) {
+                    if (blk0 + b < nblk) {
+#pragma unroll
+                        for (int e = 0; e < NF; e++) sumf[e] = sumf[e] + ex[half][(b * NR + NF * q + e) * 64 + lane];
                     }
+                }
+#pragma unroll
+                for (int e = 0; e < NB * NR; e++) acc[e] = 0.0f;
+            }
+        }
     };
     // whole groups of PD stages, then the rest: without an exit inside the loop
     // every wait leaves the later stages' loads in flight
@@ -184,24 +189,30 @@ __global__ __launch_bounds__(kOrdThreads, 4) void ordered_kernel(const OrderedAr
     for (int p = 0; p < PD - 1; p++)
         if (st + p < nst) step(st + p, p);
 
-    // chain types: t = chain l + chain l+4, then (t0 + t2) + (t1 + t3)
+    // chain types: t = chain l + chain l+4, then (t0 + t2) + (t1 + t3); with four
+    // blocks wave q holds t_q and t_{q+2}, so their sum is its own
     if constexpr (!Q8) {
 #pragma unroll
-        for (int e = 0; e < 16; e++) ex[(q * NR + e) * 64 + lane] = acc[e] + acc[16 + e];
+        for (int e = 0; e < NR; e++) {
+            float t = acc[e] + acc[NR + e];
+            if constexpr (S == 16) t = t + (acc[2 * NR + e] + acc[3 * NR + e]);
+            ex[half][(q * NR + e) * 64 + lane] = t;
+        }
         __syncthreads();
     }
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int e = 4 * q + u;  // result register of the MFMA layout
+    for (int u = 0; u < NF; u++) {
+        const int e = NF * q + u;  // result register of the MFMA layout
         float res;
         if constexpr (Q8) {
             res = sumf[u];
         } else {
-            const float* p = ex + e * 64 + lane;
-            res = (p[0] + p[2 * NR * 64]) + (p[NR * 64] + p[3 * NR * 64]);
+            const float* p = ex[half] + e * 64 + lane;
+            if constexpr (S == 32) res = (p[0] + p[2 * NR * 64]) + (p[NR * 64] + p[3 * NR * 64]);
+            else res = p[0] + p[NR * 64];
         }
-        const int tok = t0 + 8 * q + 4 * hb + u;
-        const int r = r0 + l32;
+        const int tok = t0 + (S == 32 ? 8 * (e >> 2) + 4 * blk_l + (e & 3) : 4 * blk_l + e);
+        const int r = r0 + li;
         if (tok < a.n_tok && r < a.rows) {
             const uint8_t* bias = a.b[mat];
             a.out[mat][(size_t)tok * a.ldo + r] = bias ? res + ord_bias(bias, a.bt[mat], r) : res;
@@ -209,32 +220,11 @@ __global__ __launch_bounds__(kOrdThreads, 4) void ordered_kernel(const OrderedAr
     }
 }
 
-// Image of src [rows][ld] (n columns used; any 4-byte alignment), a workgroup per
-// tile and four stages (Q8_0: a round). Rows past the last repeat it, columns
-// past n are zero.
 template <bool Q8>
 __global__ __launch_bounds__(kOrdThreads) void ordered_image_kernel(const float* __restrict__ src, int ld, int rows,
                                                                     int n, float* __restrict__ dst) {
     __shared__ __attribute__((aligned(16))) float img[4 * kOrdStageF];
-    const int tid = threadIdx.x;
-    const int nst = ord_stages(Q8, n), st0 = 4 * (int)blockIdx.x, ns = min(4, nst - st0);
-    // thread = column: the tile's rows one after the other, 1 KB of a row at a time
-    const int k = kOrdK * st0 + tid;
-    float v[kOrdTile];
-#pragma unroll
-    for (int r = 0; r < kOrdTile; r++) {
-        const int row = min((int)blockIdx.y * kOrdTile + r, rows - 1);
-        v[r] = k < n ? src[(size_t)row * ld + k] : 0.0f;
-    }
-#pragma unroll
-    for (int r = 0; r < kOrdTile; r++) {
-        int st, f;
-        ord_place(Q8, k, r, st, f);
-        img[(st - st0) * kOrdStageF + f] = v[r];
-    }
-    __syncthreads();
-    floatx4* o = (floatx4*)(dst + ((size_t)blockIdx.y * nst + st0) * kOrdStageF);
-    for (int i = tid; i < ns * kOrdStageF / 4; i += kOrdThreads) o[i] = ((const floatx4*)img)[i];
+    ordered_image_tile<Q8>(src, ld, rows, n, dst, (int)blockIdx.x, (int)blockIdx.y, img);
 }
 
 // Q8_0 rows -> the int8 values as floats [rows][n] and the block scales
@@ -285,7 +275,7 @@ hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, i
 }
 
 hipError_t launch_ordered_project(const OrderedProj* p, int nmat, int rows, int n, const float* x_image, int n_tok,
-                                  int ldo, hipStream_t s) {
+                                  int ldo, int cu_count, hipStream_t s) {
     if (rows <= 0 || n_tok <= 0 || n <= 0 || n % 8 || nmat < 1 || nmat > 2) return hipErrorInvalidValue;
     const bool q8 = p[0].type == GG_Q8_0;
     if (q8 && n % 32) return hipErrorInvalidValue;
@@ -305,9 +295,21 @@ hipError_t launch_ordered_project(const OrderedProj* p, int nmat, int rows, int 
     a.n = n;
     a.ldo = ldo;
     a.rtiles = (rows + kOrdTile - 1) / kOrdTile;
-    const dim3 grid((unsigned)(a.rtiles * nmat), (unsigned)((n_tok + kOrdTile - 1) / kOrdTile));
-    if (q8) hipLaunchKernelGGL(ordered_kernel<true>, grid, dim3(kOrdThreads), 0, s, a);
-    else hipLaunchKernelGGL(ordered_kernel<false>, grid, dim3(kOrdThreads), 0, s, a);
+    // 16 x 16 tiles where 32 x 32 ones leave SIMDs idle or with a lone wave (which
+    // adds at half the rate): 75 tokens x 2 x 1024 rows x 2560 34 -> 26 us, 10 tokens
+    // 34 -> 19; from the second wave per SIMD on both take the same time
+    const long long wgs = (long long)a.rtiles * nmat * ((n_tok + kOrdTile - 1) / kOrdTile);
+    const int S = wgs <= cu_count ? 16 : 32;
+    const dim3 grid((unsigned)(a.rtiles * nmat), (unsigned)((n_tok + S - 1) / S));
+#define PQA_ORD(Q, SS) hipLaunchKernelGGL((ordered_kernel<Q, SS>), grid, dim3(kOrdThreads), 0, s, a)
+    if (q8) {
+        if (S == 16) PQA_ORD(true, 16);
+        else PQA_ORD(true, 32);
+    } else {
+        if (S == 16) PQA_ORD(false, 16);
+        else PQA_ORD(false, 32);
+    }
+#undef PQA_ORD
     return hipGetLastError();
 }
 

@@ -183,6 +183,17 @@ hipError_t launch_gemm_f16x3_nt(const GemmPlan& plan, const _Float16* a, int lda
                                 int ldc, size_t slice_stride, int m, int n, int kh, hipStream_t stream);
 hipError_t launch_prefill(pqa_ctx* ctx, int layer, int start, int n_tok, const float* q,
                           const float* k, const float* v, float* out);
+// y[t * ld + c] = the sum of a GEMM's K slices part[s * stride + t * cols + c] in slice
+// order, c < cols (an even number), t < n_tok
+struct SliceSum {
+    const float* part;
+    float* y;
+    size_t stride;
+    int slices, cols, ld, n_tok;
+};
+inline long long sum_slices_blocks(const SliceSum& a) { return ((long long)a.n_tok * (a.cols / 2) + 255) / 256; }
+hipError_t launch_sum_slices(const SliceSum& a, hipStream_t s);
+
 // q/k/v of a prompt as the columns of one GEMM result y [n_tok][ld] (q at
 // column 0, k at q_dim, v at q_dim + kv_dim), scaled by powers of two: the
 // value of column c of token t is y * (w_inv[c] * x_inv[t]) + b_m[c]
@@ -196,6 +207,9 @@ struct PrefillScaled {
     const uint8_t* b[3];  // q, k, v biases or null
     int bt[3];
     bool kv_plain;
+    // slices > 0: the q columns of y are still to be summed, before the attention
+    // (and, as it happens, in the same launch as the K/V prep)
+    SliceSum sum;
 };
 hipError_t launch_prefill_scaled(pqa_ctx* ctx, int layer, int start, int n_tok, const PrefillScaled& ys, float* out);
 // The general-head_dim path (pqa_general.hip): the same contracts as
@@ -231,7 +245,7 @@ hipError_t prepare_exact_matrix(int type, const void* w, int stride, int rows, i
                                 hipStream_t s);
 hipError_t launch_ordered_image(bool q8, const float* src, int ld, int rows, int n, float* dst, hipStream_t s);
 hipError_t launch_ordered_project(const OrderedProj* p, int nmat, int rows, int n, const float* x_image, int n_tok,
-                                  int ldo, hipStream_t s);
+                                  int ldo, int cu_count, hipStream_t s);
 hipError_t launch_out_project(pqa_ctx* ctx, int layer, const float* attn, float* x);
 
 }  // namespace pqa

@@ -55,6 +55,9 @@ struct KvArgs {
     const uint8_t* kb;
     const uint8_t* vb;
     int kbt, vbt;
+    // workgroups past kv_blocks sum the GEMM's K slices of the q columns
+    int kv_blocks;
+    SliceSum sum;
 };
 
 // y * (w * xi) + b[c .. c+3] (an exact power-of-two rescale, then vec_add,
@@ -99,6 +102,10 @@ __global__ __launch_bounds__(kKvThreads) void prefill_kv_kernel(const KvArgs a) 
     constexpr int RS = HD + 4;        // LDS row stride in floats (rows r and r + 8 share banks: 2-way)
     __shared__ __attribute__((aligned(16))) float sk[NW][RPW * RS];
     __shared__ float s_scale[NW][RPW];
+    if ((int)blockIdx.x >= a.kv_blocks) {
+        sum_slices(a.sum, (int)blockIdx.x - a.kv_blocks);
+        return;
+    }
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int t = lane % H4, hh = lane / H4;
@@ -1026,7 +1033,9 @@ static hipError_t launch_prefill_hd(pqa_ctx* ctx, int layer, int start, int n_to
     }
     constexpr int rows_per_wg = (kKvThreads / 64) * kv_rows_per_wave<HD>();
     const int n_items = n_tok * ctx->n_kv_heads;
-    const dim3 kv_grid((n_items + rows_per_wg - 1) / rows_per_wg);
+    p.kv_blocks = (n_items + rows_per_wg - 1) / rows_per_wg;
+    p.sum = YS ? ys->sum : SliceSum{};
+    const dim3 kv_grid((unsigned)(p.kv_blocks + (p.sum.slices ? sum_slices_blocks(p.sum) : 0)));
     if (kv_scaled)
         hipLaunchKernelGGL((prefill_kv_kernel<HD, true>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
     else
@@ -1101,6 +1110,10 @@ hipError_t launch_prefill_scaled(pqa_ctx* ctx, int layer, int start, int n_tok, 
         return launch_prefill_hd<64, true>(ctx, layer, start, n_tok, nullptr, nullptr, nullptr, out, &ys);
     if (ctx->head_dim == 128)
         return launch_prefill_hd<128, true>(ctx, layer, start, n_tok, nullptr, nullptr, nullptr, out, &ys);
+    if (ys.sum.slices) {
+        const hipError_t e = launch_sum_slices(ys.sum, ctx->stream);
+        if (e != hipSuccess) return e;
+    }
     return launch_prefill_general(ctx, layer, start, n_tok, nullptr, nullptr, nullptr, &ys, out);
 }
 
