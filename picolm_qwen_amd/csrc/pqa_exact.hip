@@ -37,10 +37,11 @@
 // 16-byte loads each per stage, requested two stages ahead (one for Q8_0). At the
 // end (Q8_0: of each round) the waves' sums meet in LDS and each wave finishes a
 // quarter of the tile in the reference's order.
-// K and V together, 2 x 1024 rows x 2560: 2048 tokens 353 us and 9 for the inputs'
-// image (a 64 x 64 register tile with VALU multiplies, a launch each: 506 us); 75
-// tokens 35 + 5 us (226 us). 2048 tokens run at 163 cycles per MFMA and its 32
-// additions, against 152 measured for the two alone.
+// Short prompts run 16 x 16 tiles with four sequences per wave (below).
+// K and V together, 2 x 1024 rows x 2560: 2048 tokens 353 us (a 64 x 64 register
+// tile with VALU multiplies, a launch each: 506 us), 75 tokens 26 us (226 us). 2048
+// tokens run at 163 cycles per MFMA and its 32 additions, against 141 measured for
+// the two alone at four waves per SIMD.
 //
 // Image of a matrix [rows][n] (n rounded up to whole stages, Q8_0 whole rounds,
 // with zeros): per tile of 32 rows and stage, [wave q][half h][lane][4]: lane l is

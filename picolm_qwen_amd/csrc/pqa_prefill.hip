@@ -55,7 +55,7 @@ struct KvArgs {
     const uint8_t* kb;
     const uint8_t* vb;
     int kbt, vbt;
-    // workgroups past kv_blocks sum the GEMM's K slices of the q columns
+    // SUM
     int kv_blocks;
     SliceSum sum;
 };
@@ -91,7 +91,9 @@ constexpr int kKvRowsPerWave = PQA_KV_ROWS_PER_WAVE;
 template <int HD>
 constexpr int kv_rows_per_wave() { return kKvRowsPerWave < 256 / HD ? 256 / HD : kKvRowsPerWave; }
 
-template <int HD, bool YS>
+// SUM: workgroups past kv_blocks sum the GEMM's K slices of the q columns, which
+// nothing reads before the next launch.
+template <int HD, bool YS, bool SUM>
 __global__ __launch_bounds__(kKvThreads) void prefill_kv_kernel(const KvArgs a) {
     constexpr int H4 = HD / 4;        // lanes per row
     constexpr int RPS = 64 / H4;      // rows per slot
@@ -102,9 +104,11 @@ __global__ __launch_bounds__(kKvThreads) void prefill_kv_kernel(const KvArgs a) 
     constexpr int RS = HD + 4;        // LDS row stride in floats (rows r and r + 8 share banks: 2-way)
     __shared__ __attribute__((aligned(16))) float sk[NW][RPW * RS];
     __shared__ float s_scale[NW][RPW];
-    if ((int)blockIdx.x >= a.kv_blocks) {
-        sum_slices(a.sum, (int)blockIdx.x - a.kv_blocks);
-        return;
+    if constexpr (SUM) {
+        if ((int)blockIdx.x >= a.kv_blocks) {
+            sum_slices(a.sum, (int)blockIdx.x - a.kv_blocks);
+            return;
+        }
     }
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
@@ -952,7 +956,7 @@ static int prefill_ranges(int start, int n_tok, int g, int n_kv, int nblk, int c
     const size_t rows = (size_t)n_tok * g * n_kv;
     for (int s = 1; s <= 16 && s <= 2 * longest; s++) {
         if (s > 1 && s * rows > max_rows) break;
-        const double combine = s > 1 ? 4.0 + s * (double)rows / 2e4 : 0.0;
+        const double combine = s > 1 ? 6.0 + s * (double)rows / 2e4 : 0.0;
         const double t = rounds((long long)nblk * n_kv * s) * ((double)longest / s + block) + combine;
         if (t < best) {
             best = t;
@@ -1036,10 +1040,12 @@ static hipError_t launch_prefill_hd(pqa_ctx* ctx, int layer, int start, int n_to
     p.kv_blocks = (n_items + rows_per_wg - 1) / rows_per_wg;
     p.sum = YS ? ys->sum : SliceSum{};
     const dim3 kv_grid((unsigned)(p.kv_blocks + (p.sum.slices ? sum_slices_blocks(p.sum) : 0)));
-    if (kv_scaled)
-        hipLaunchKernelGGL((prefill_kv_kernel<HD, true>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
+    if (kv_scaled)  // (its slices are summed before)
+        hipLaunchKernelGGL((prefill_kv_kernel<HD, true, false>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
+    else if (p.sum.slices)
+        hipLaunchKernelGGL((prefill_kv_kernel<HD, false, true>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
     else
-        hipLaunchKernelGGL((prefill_kv_kernel<HD, false>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
+        hipLaunchKernelGGL((prefill_kv_kernel<HD, false, false>), kv_grid, dim3(kKvThreads), 0, ctx->stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
 

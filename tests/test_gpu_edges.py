@@ -207,3 +207,20 @@ def test_general_mma_non_finite_rows(hd):
     dec = att.forward(0, t, *(torch.from_numpy(x[t]).to(DEV) for x in (q, k, v))).cpu().numpy()
     assert np.array_equal(np.isnan(dec), np.isnan(want)) and np.array_equal(np.isinf(dec), np.isinf(want))
     att.close()
+
+
+# prompts with enough 32 x 32 tiles for two waves per SIMD (the smaller ones above run 16 x 16)
+@pytest.mark.parametrize("kt,vt,dim", [(O.GGUF_Q8_0, O.GGUF_Q8_0, 320), (O.GGUF_F16, O.GGUF_F16, 136)])
+def test_ordered_projection_many_tiles(kt, vt, dim):
+    print(f"reference-order K/V, 270 tokens x 2 x 1024 rows, types {kt}/{vt}, width {dim}", flush=True)
+    rng = np.random.default_rng(dim)
+    nkv, hd, n_tok = 8, 128, 270
+    att = PicoAttention(1, 16, nkv, nkv, hd)
+    rows = nkv * hd
+    w = [make_rows(rng, t, rows, dim) for t in (kt, kt, vt)]
+    att.set_qkv_weights(0, dim, w[0], kt, w[1], kt, w[2], vt)
+    x = rng.standard_normal((n_tok, dim)).astype(np.float32)
+    _, k, v = (g.cpu().numpy() for g in att.qkv_project_batch(0, torch.from_numpy(x).to(DEV)))
+    assert_bits_equal(_bits(k), _bits(O.matmul_bias_tokens(x, w[1], kt, rows)), "k")
+    assert_bits_equal(_bits(v), _bits(O.matmul_bias_tokens(x, w[2], vt, rows)), "v")
+    att.close()
