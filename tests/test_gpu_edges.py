@@ -224,3 +224,16 @@ def test_ordered_projection_many_tiles(kt, vt, dim):
     assert_bits_equal(_bits(k), _bits(O.matmul_bias_tokens(x, w[1], kt, rows)), "k")
     assert_bits_equal(_bits(v), _bits(O.matmul_bias_tokens(x, w[2], vt, rows)), "v")
     att.close()
+
+
+# the same through the host entries, whose decode reads q, k and v and writes out in pinned host memory
+@pytest.mark.parametrize("hd", [80, 256])
+def test_general_mma_host_decode(hd):
+    print(f"general decode from host memory, hd {hd}", flush=True)
+    nh, nkv, pos, seed = 6, 2, 700, 5400 + hd
+    att, q, k, v, qn, kn, cos, sin, kc, vc = _gen_case(hd, nh, nkv, pos, 1, 0, seed)
+    dev = att.forward(0, pos, *(torch.from_numpy(x[0]).to(DEV) for x in (q, k, v))).cpu().numpy()
+    out = np.asarray(att.forward(0, pos, q[0], k[0], v[0]))
+    assert_bits_equal(_bits(out), _bits(dev), "host against device entry")
+    _check_gen(att, O.shape(nh, nkv, hd, pos + 1, 0), pos, [0], out[None], q, k, v, qn, kn, cos, sin, kc, vc)
+    att.close()
