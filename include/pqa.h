@@ -271,7 +271,12 @@ int pqa_attention_block(pqa_ctx* ctx, int layer, int pos, const float* xb, float
  * replaced or the context is destroyed; the first call also allocates a
  * q_dim * n_embd float workspace, and each call needs a workspace of about
  * n_tok * (4 n_embd + 4 (q_dim + 2 kv_dim) + 4) bytes (the hi and lo halves
- * of a row each padded to 32 halfs), grown on demand.
+ * of a row each padded to 32 halfs), another 4 n_embd for each of n_tok
+ * rounded up to 32 (the inputs' image; n_embd rounded up to 64, for Q8_0 rows
+ * to 256), and the smaller of 64 n_tok (q_dim + 2 kv_dim) bytes and 192 KiB
+ * per CU (50 MB) for the GEMM's K slices. It is grown on demand and depends on
+ * n_tok alone, never less for more tokens: after one call with the longest
+ * prompt, shorter ones allocate nothing and a captured call keeps its buffers.
  */
 int pqa_qkv_project_batch(pqa_ctx* ctx, int layer, int n_tok, const float* xb, float* q, float* k, float* v);
 

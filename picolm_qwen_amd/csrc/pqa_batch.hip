@@ -475,50 +475,46 @@ struct SplitBufs {
     float* image;  // of X, for the reference-order projection
 };
 
-// Bytes of one batched product's buffers: y_floats of result, part_floats of K
-// slices and an image of image floats.
-static size_t split_need(int n_tok, int n, size_t y_floats, size_t part_floats, size_t image) {
-    return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2) + up256((size_t)n_tok * 4) + up256(y_floats * 4) +
-           up256(part_floats * 4) + image * 4;
+// The buffers of one batched product over n_tok inputs of n elements: y_floats of
+// result, part_floats of K slices and an image of image floats. None depends on what
+// the GEMM's plan picks for n_tok, and each grows with n_tok, so a call with the
+// longest prompt makes the workspace of every shorter one (nothing is allocated in a
+// capture of one, and no captured launch loses its buffers to one).
+struct BatchShape {
+    int n_tok, n;
+    size_t y_floats, part_floats, image;
+
+    size_t x_bytes() const { return up256((size_t)n_tok * 2 * pqa::k_half(n) * 2); }
+    size_t bytes() const {
+        return x_bytes() + up256((size_t)n_tok * 4) + up256(y_floats * 4) + up256(part_floats * 4) + image * 4;
+    }
+};
+
+// The q/k/v product, whether K and V run on the GEMM or in the reference's order
+static BatchShape qkv_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok) {
+    const size_t total = ctx->q_dim + 2 * ctx->kv_dim;
+    return BatchShape{n_tok, p.n_embd, (size_t)n_tok * total, pqa::gemm_slice_floats(n_tok, (int)total, ctx->cu_count),
+                      image_floats(p, n_tok)};
+}
+// The output product, whose slices the residual kernel sums
+static BatchShape out_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok) {
+    const size_t y = std::max((size_t)n_tok * p.out_rows, pqa::gemm_slice_floats(n_tok, p.out_rows, ctx->cu_count));
+    return BatchShape{n_tok, (int)ctx->q_dim, y, 0, 0};
 }
 
-static int ensure_split(pqa_ctx* ctx, int n_tok, int n, size_t y_floats, size_t part_floats, size_t image,
-                        SplitBufs* sb, const char* fn) {
-    if (int rc = grow_split(ctx, split_need(n_tok, n, y_floats, part_floats, image), fn)) return rc;
+static int ensure_split(pqa_ctx* ctx, const BatchShape& b, SplitBufs* sb, const char* fn) {
+    if (int rc = grow_split(ctx, b.bytes(), fn)) return rc;
     char* base = (char*)ctx->bsplit;
     sb->x3 = (_Float16*)base;
-    base += up256((size_t)n_tok * 2 * pqa::k_half(n) * 2);
+    base += b.x_bytes();
     sb->x_inv = (float*)base;
-    base += up256((size_t)n_tok * 4);
+    base += up256((size_t)b.n_tok * 4);
     sb->y = (float*)base;
-    base += up256(y_floats * 4);
+    base += up256(b.y_floats * 4);
     sb->parts = (float*)base;
-    base += up256(part_floats * 4);
+    base += up256(b.part_floats * 4);
     sb->image = (float*)base;
     return PQA_OK;
-}
-
-// The buffers of the q/k/v product (q_only: the GEMM covers the q columns alone
-// and the reference-order projection needs an image) and of the output product.
-struct BatchShape {
-    pqa::GemmPlan plan;
-    size_t y_floats, part_floats, image;
-};
-static BatchShape qkv_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok, bool q_only) {
-    const size_t total = ctx->q_dim + 2 * ctx->kv_dim, cols = q_only ? ctx->q_dim : total;
-    BatchShape b;
-    b.plan = pqa::gemm_f16x3_plan(n_tok, (int)cols, pqa::k_half(p.n_embd), ctx->cu_count);
-    b.y_floats = (size_t)n_tok * total;
-    b.part_floats = b.plan.slices > 1 ? (size_t)b.plan.slices * n_tok * cols : 0;
-    b.image = q_only ? image_floats(p, n_tok) : 0;
-    return b;
-}
-static BatchShape out_shape(const pqa_ctx* ctx, const pqa_proj_weights& p, int n_tok) {
-    BatchShape b;
-    b.plan = pqa::gemm_f16x3_plan(n_tok, p.out_rows, pqa::k_half((int)ctx->q_dim), ctx->cu_count);
-    b.y_floats = (size_t)b.plan.slices * n_tok * p.out_rows;  // the residual kernel sums the slices
-    b.part_floats = b.image = 0;
-    return b;
 }
 
 // X' and the GEMM of one call: sb->y [n_tok][q_dim + 2 kv_dim] = X W^T, every
@@ -536,8 +532,7 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
     const int kh = pqa::k_half(n);
     const _Float16* w3 = (const _Float16*)p.split;
     *w_inv = (const float*)((const char*)p.split + up256(total * 2 * kh * 2));
-    const BatchShape bs = qkv_shape(ctx, p, n_tok, q_only);
-    if (int rc = ensure_split(ctx, n_tok, n, bs.y_floats, bs.part_floats, bs.image, sb, fn)) return rc;
+    if (int rc = ensure_split(ctx, qkv_shape(ctx, p, n_tok), sb, fn)) return rc;
     if (q_only) {
         const hipError_t e = pqa::launch_split2_image(xb, n_tok, n, sb->x3, kh, sb->x_inv, p.wtype[1] == pqa::GG_Q8_0,
                                                       sb->image, ctx->stream);
@@ -548,13 +543,14 @@ static int batch_gemm(pqa_ctx* ctx, int layer, int n_tok, const float* xb, Split
     }
     // Y[n_tok][total] = X_hi W_hi^T + X_hi W_lo^T + X_lo W_hi^T (the q rows come first)
     const int cols = q_only ? (int)ctx->q_dim : (int)total;
-    const bool sliced = bs.plan.slices > 1;
+    const pqa::GemmPlan plan = pqa::gemm_f16x3_plan(n_tok, cols, kh, ctx->cu_count);
+    const bool sliced = plan.slices > 1;
     const size_t stride = (size_t)n_tok * cols;
     const hipError_t e =
-        pqa::launch_gemm_f16x3_nt(bs.plan, sb->x3, 2 * kh, w3, 2 * kh, sliced ? sb->parts : sb->y,
+        pqa::launch_gemm_f16x3_nt(plan, sb->x3, 2 * kh, w3, 2 * kh, sliced ? sb->parts : sb->y,
                                   sliced ? cols : (int)total, stride, n_tok, cols, kh, ctx->stream);
     if (int rc = hip_check(ctx, e, fn)) return rc;
-    *sum = pqa::SliceSum{sb->parts, sb->y, stride, sliced ? bs.plan.slices : 0, cols, (int)total, n_tok};
+    *sum = pqa::SliceSum{sb->parts, sb->y, stride, sliced ? plan.slices : 0, cols, (int)total, n_tok};
     return PQA_OK;
 }
 
@@ -655,22 +651,22 @@ static int out_project_batch(pqa_ctx* ctx, int layer, int n_tok, const float* at
     const auto& p = ctx->proj[layer];
     const int n = (int)ctx->q_dim, rows = p.out_rows;
     const int kh = pqa::k_half(n);
-    const BatchShape bs = out_shape(ctx, p, n_tok);
+    const pqa::GemmPlan plan = pqa::gemm_f16x3_plan(n_tok, rows, kh, ctx->cu_count);
     SplitBufs sb;
-    if (int rc = ensure_split(ctx, n_tok, n, bs.y_floats, 0, 0, &sb, fn)) return rc;
+    if (int rc = ensure_split(ctx, out_shape(ctx, p, n_tok), &sb, fn)) return rc;
     pqa::launch_split2(attn, n_tok, n, sb.x3, kh, sb.x_inv, ctx->stream);
     if (int rc = hip_check(ctx, hipGetLastError(), fn)) return rc;
     const _Float16* w3 = (const _Float16*)p.out_split;
     const float* w_inv = (const float*)((const char*)p.out_split + up256((size_t)rows * 2 * kh * 2));
     const size_t stride = (size_t)n_tok * rows;
     if (int rc = hip_check(ctx,
-                           pqa::launch_gemm_f16x3_nt(bs.plan, sb.x3, 2 * kh, w3, 2 * kh, sb.y, rows, stride, n_tok,
+                           pqa::launch_gemm_f16x3_nt(plan, sb.x3, 2 * kh, w3, 2 * kh, sb.y, rows, stride, n_tok,
                                                      rows, kh, ctx->stream),
                            fn))
         return rc;
     const unsigned gx = (unsigned)((rows / 4 + 255) / 256);
     hipLaunchKernelGGL(pqa::unscale_residual_kernel, dim3(gx, n_tok), dim3(256), 0, ctx->stream, (const float*)sb.y,
-                       bs.plan.slices, stride, rows, w_inv, (const float*)sb.x_inv, (const uint8_t*)p.b[3],
+                       plan.slices, stride, rows, w_inv, (const float*)sb.x_inv, (const uint8_t*)p.b[3],
                        p.btype[3], x);
     return hip_check(ctx, hipGetLastError(), fn);
 }
@@ -707,9 +703,7 @@ extern "C" int pqa_prefill_block(pqa_ctx* ctx, int layer, int start_pos, int n_t
         return set_err(ctx, PQA_ERR_RANGE, "pqa_prefill_block: positions past max_seq_len");
     // every buffer of both GEMMs exists before the first kernel is queued
     const auto& p = ctx->proj[layer];
-    const BatchShape bq = qkv_shape(ctx, p, n_tok, ctx->batch_exact_kv != 0), bo = out_shape(ctx, p, n_tok);
-    const size_t need = std::max(split_need(n_tok, p.n_embd, bq.y_floats, bq.part_floats, bq.image),
-                                 split_need(n_tok, (int)ctx->q_dim, bo.y_floats, 0, 0));
+    const size_t need = std::max(qkv_shape(ctx, p, n_tok).bytes(), out_shape(ctx, p, n_tok).bytes());
     if (int rc = grow_split(ctx, need, fn)) return rc;
     const size_t af = (size_t)n_tok * ctx->q_dim;
     if (af > ctx->battn_floats) {

@@ -34,8 +34,6 @@
 // (at 2048 x 6144: 8 m-blocks x 4 n-blocks per XCD).
 //
 // Rows past m (n) load the last row (clamped, never stored).
-#include <algorithm>
-
 #include "pqa_device.h"
 #include "pqa_internal.h"
 
@@ -43,7 +41,7 @@ namespace pqa {
 
 constexpr int kGemmWaves = 4;
 constexpr int kGemmThreads = 64 * kGemmWaves;
-constexpr int kG3BK = 32;
+constexpr int kG3BK = kGemmBK;
 constexpr int kG3RowB = kG3BK * 2;  // 64 bytes per tile row
 
 template <int N>
@@ -256,45 +254,6 @@ static hipError_t launch_g3(Gemm3Args g, hipStream_t stream) {
     if (groups > 0x7FFFFFFF) return hipErrorInvalidValue;
     hipLaunchKernelGGL((gemm_f16x3_nt_kernel<MI, NJ, NS>), dim3((unsigned)groups), dim3(kGemmThreads), 0, stream, g);
     return hipGetLastError();
-}
-
-// The tile and K slices with the least expected time, in us, from rates measured
-// over 110 shapes (2 to 2048 rows, 896 to 6144 columns, K 896 to 4096; the pick is
-// 3.5 % off the fastest of all combinations on average). A k tile takes a
-// workgroup `step` when it has a CU for itself, and the chip as a whole needs
-// `flow` per k tile and 32 x 32 block (operand traffic and power, 1.1-1.2 PFLOP/s
-// on the two largest tiles); each round of workgroups costs a pipeline fill, and
-// slices the launch that sums them and their way through memory. Against the one
-// 256 x 192 tile without slices: 75 x 4096 x 2560 115 -> 17 us, 75 x 2560 x 4096
-// 163 -> 16, 2048 x 4096 x 2560 138 -> 118 (256 x 128: 256 tiles on 256 CUs where
-// 176 were busy), 2048 x 2560 x 4096 192 -> 129 (two slices of 112 tiles).
-GemmPlan gemm_f16x3_plan(int m, int n, int kh, int cu_count) {
-    static const struct {
-        int mi, nj, occupancy;
-        double step, flow;
-    } tiles[] = {{4, 3, 1, 1.45, 6.2e-4}, {4, 2, 1, 1.08, 6.3e-4}, {2, 2, 2, 0.66, 6.5e-4}, {2, 1, 2, 0.35, 7.3e-4},
-                 {1, 1, 2, 0.25, 8.5e-4}};
-    const int ktiles = std::max(1, kh / kG3BK);
-    const double cus = cu_count;
-    GemmPlan best{4, 3, 1};
-    double best_us = 1e30;
-    for (const auto& t : tiles) {
-        const long long mn = (long long)((m + 64 * t.mi - 1) / (64 * t.mi)) * ((n + 64 * t.nj - 1) / (64 * t.nj));
-        for (int s = 1; s <= 16 && s <= ktiles; s++) {
-            const long long wgs = mn * s;
-            if (s > 1 && wgs > 4LL * cu_count) break;
-            const double kt = (double)ktiles / s;
-            const double alone = (double)((wgs + cu_count - 1) / cu_count) * kt * t.step;
-            const double chip = (double)wgs * kt * t.mi * t.nj * t.flow * (256.0 / cus);
-            double us = std::max(alone, chip) + std::max(1.0, (double)wgs / (cus * t.occupancy));
-            if (s > 1) us += 3.0 + (2.0 * s + 1.0) * m * (double)n * 4e-6 / 5.5;
-            if (us < best_us) {
-                best_us = us;
-                best = GemmPlan{t.mi, t.nj, s};
-            }
-        }
-    }
-    return best;
 }
 
 hipError_t launch_gemm_f16x3_nt(const GemmPlan& plan, const _Float16* a, int lda, const _Float16* b, int ldb, float* c,

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "pqa.h"
+#include "pqa_gemm_plan.h"
 
 #define PQA_MAX_EMBD 8192  // longest projection input row (x and the chunk rings share the LDS)
 
@@ -172,13 +173,8 @@ int scratch_init(int device);
 int scratch_workspace(pqa_ctx* ctx, DecodeWorkspace* ws, const char* fn);
 // C[m][n] = A_hi B_hi^T + A_hi B_lo^T + A_lo B_hi^T with rows of A (B) holding
 // hi at [0, kh) and lo at [kh, 2 kh) halfs (fp16 operands, fp32 result; kh a
-// multiple of 32; pqa_gemm.hip). The plan is the workgroup tile (64 mi x 64 nj)
-// and the number of K slices: slice i's part of the sum is stored at c + i *
-// slice_stride, and C is the sum over the slices.
-struct GemmPlan {
-    int mi, nj, slices;
-};
-GemmPlan gemm_f16x3_plan(int m, int n, int kh, int cu_count);
+// multiple of 32; pqa_gemm.hip). Slice i of the plan's K slices is stored at c +
+// i * slice_stride, and C is the sum over the slices.
 hipError_t launch_gemm_f16x3_nt(const GemmPlan& plan, const _Float16* a, int lda, const _Float16* b, int ldb, float* c,
                                 int ldc, size_t slice_stride, int m, int n, int kh, hipStream_t stream);
 hipError_t launch_prefill(pqa_ctx* ctx, int layer, int start, int n_tok, const float* q,

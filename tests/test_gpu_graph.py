@@ -115,3 +115,50 @@ def test_graph_replays_equal_eager_prefill():
             assert np.array_equal(gk, rows[layer][0]) and np.array_equal(gv, rows[layer][1]), (rep, layer)
     g.close()
     att.close()
+
+
+def test_shorter_prompt_after_a_longer_one_needs_no_new_workspace():
+    # a warm-up with the longest prompt covers every shorter one, also where the shorter one's GEMMs
+    # are cut into K slices and the longer one's are not (137 tokens, 4 slices; 138, one): its capture
+    # allocates nothing, and the longer prompt's graph keeps its buffers, in both K/V projection modes
+    print("graph prompt blocks, 138 then 137 and 20 tokens", flush=True)
+    rng = np.random.default_rng(9300)
+    nh, nkv, hd, dim, smax = 32, 8, 128, 2560, 160
+    att = PicoAttention(1, smax, nh, nkv, hd, 0)
+    w = [(rng.standard_normal((r, n), dtype=np.float32) / np.sqrt(n)).astype(np.float16).view(np.uint8)
+         for r, n in ((nh * hd, dim), (nkv * hd, dim), (nkv * hd, dim), (dim, nh * hd))]
+    att.set_qkv_weights(0, dim, *(a for m in w[:3] for a in (m, O.GGUF_F16)))
+    att.set_out_weights(0, dim, w[3], O.GGUF_F16)
+    L = _lib.lib()
+    stream = L.pqa_stream(att.handle)
+    for exact_kv in (True, False):
+        att.set_batch_projection(exact_kv)
+        runs = []
+        for n in (138, 137, 20):
+            xb = torch.from_numpy(rng.standard_normal((n, dim)).astype(np.float32)).to(DEV)
+            runs.append([n, xb, torch.zeros(n, dim, device=DEV), None, None])
+        torch.cuda.synchronize()
+
+        def block(run):
+            assert L.pqa_prefill_block(att.handle, 0, 0, run[0], _ptr(run[1]), _ptr(run[2])) == 0, att.last_error()
+
+        block(runs[0])  # the longest prompt, once
+        att.sync()
+        for run in runs:
+            run[3] = Graph(stream, lambda: block(run))
+        for run in runs:
+            run[2].zero_()
+            torch.cuda.synchronize()
+            block(run)
+            att.sync()
+            run[4] = run[2].clone()
+        for rep in range(3):
+            for run in runs:
+                run[2].zero_()
+                torch.cuda.synchronize()
+                run[3].launch(stream)
+                att.sync()
+                assert torch.equal(run[2].view(torch.int32), run[4].view(torch.int32)), (exact_kv, run[0], rep)
+        for run in runs:
+            run[3].close()
+    att.close()
