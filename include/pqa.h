@@ -58,7 +58,10 @@ typedef enum {
  * plain VALU kernels with the same results contract (bit-exact K/V rows,
  * outputs within max-abs 2e-3 / rel 1e-2), where q, k and v need only 4-byte
  * and out 8-byte alignment. The cache starts zeroed, as the reference's
- * std::vector does.
+ * std::vector does. Besides the cache and the tables the context holds its
+ * workspaces, the largest for the key ranges of a prompt: up to 256 rows of
+ * head_dim + 2 floats per CU (34 MB at head size 128 on 256 CUs; 128 rows at the
+ * matrix-core sizes other than 64 and 128, none at the VALU sizes).
  */
 int pqa_create(pqa_ctx** out, int n_layers, int max_seq_len, int n_heads, int n_kv_heads,
                int head_dim, int rope_style, const float* rope_cos, const float* rope_sin);
@@ -88,7 +91,11 @@ int pqa_decode(pqa_ctx* ctx, int layer, int pos, const float* q, const float* k,
  * pointers q [n_tok][n_heads*hd], k/v [n_tok][n_kv*hd], out [n_tok][n_heads*hd].
  * Rows are appended first and attention is causal (token i reads rows
  * 0..start_pos+i), which is what the reference's serial loop computes.
- * Same alignment and readiness rules as pqa_decode.
+ * Same alignment and readiness rules as pqa_decode. Under stream capture it
+ * needs no earlier call: few tokens behind a long history, whose keys are cut
+ * into ranges, keep a buffer per layer from the first such capture on
+ * (pqa_create), so that captured prompts of different layers may be replayed
+ * at once.
  */
 int pqa_prefill(pqa_ctx* ctx, int layer, int start_pos, int n_tok, const float* q, const float* k,
                 const float* v, float* out);

@@ -39,6 +39,8 @@ static void free_ctx(pqa_ctx* c) {
     void* bufs[] = {c->key_cache, c->val_cache, c->slab, c->stage, c->gen_q};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
+    for (float* b : c->pf_captured)
+        if (b) (void)hipFree(b);
     if (c->hstage) (void)hipHostFree(c->hstage);
     for (int i = 0; i < 2; ++i) {
         if (c->kvc_buf[i]) (void)hipHostFree(c->kvc_buf[i]);

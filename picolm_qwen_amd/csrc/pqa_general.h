@@ -27,9 +27,9 @@ __device__ __forceinline__ float gen_load(const GenSrc& s, int t, int c) {
     return v;
 }
 
-// Attention of one layer on the MFMA kernels: a decode (n_tok 1; appends the new
-// row itself) or a prompt (its rows already appended).
-hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, bool decode, const GenSrc& q, const GenSrc& k,
-                          const GenSrc& v, float* out, float* part_acc, float* part_ml, size_t part_rows);
+// Attention of one layer on the MFMA kernels: a decode with ws (n_tok 1; appends the
+// new row itself) or, with ws null, a prompt (its rows already appended).
+hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, const DecodeWorkspace* ws, const GenSrc& q,
+                          const GenSrc& k, const GenSrc& v, float* out);
 
 }  // namespace pqa

@@ -550,9 +550,8 @@ static GenSrc plain_src(const float* p, size_t ld) { return GenSrc{p, (int)ld, n
 hipError_t launch_decode_general(pqa_ctx* ctx, int layer, int pos, const float* q, const float* k, const float* v,
                                  float* out, const DecodeWorkspace& ws) {
     if (gen_mma_head_dim(ctx->head_dim))
-        return launch_gen_mma(ctx, layer, pos, 1, true, plain_src(q, ctx->q_dim), plain_src(k, ctx->kv_dim),
-                              plain_src(v, ctx->kv_dim), out, ws.part_acc, ws.part_ml,
-                              (size_t)ws.max_splits * ctx->n_heads);
+        return launch_gen_mma(ctx, layer, pos, 1, &ws, plain_src(q, ctx->q_dim), plain_src(k, ctx->kv_dim),
+                              plain_src(v, ctx->kv_dim), out);
     // gen_q holds one token's q from context creation on: no allocation here
     if (ctx->gen_q_floats < ctx->q_dim) return hipErrorInvalidValue;
     hipError_t e = launch_gen_prep(ctx, layer, pos, 1, plain_src(q, ctx->q_dim), plain_src(k, ctx->kv_dim),
@@ -580,9 +579,7 @@ hipError_t launch_prefill_general(pqa_ctx* ctx, int layer, int start, int n_tok,
     }
     e = launch_gen_prep(ctx, layer, start, n_tok, sq, sk, sv, !mma);
     if (e != hipSuccess) return e;
-    if (mma)
-        return launch_gen_mma(ctx, layer, start, n_tok, false, sq, sk, sv, out, ctx->pf_part,
-                              ctx->pf_part + ctx->pf_rows * ctx->head_dim, ctx->pf_rows);
+    if (mma) return launch_gen_mma(ctx, layer, start, n_tok, nullptr, sq, sk, sv, out);
     return launch_gen_attn(ctx, layer, start, n_tok, out, nullptr);
 }
 

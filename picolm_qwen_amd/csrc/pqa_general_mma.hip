@@ -622,9 +622,11 @@ static void launch_gm(const GenMmaArgs& a, bool decode, unsigned grid, hipStream
     else hipLaunchKernelGGL((gen_mma_kernel<HD, false>), dim3(grid), dim3(256), 0, s, a);
 }
 
-hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, bool decode, const GenSrc& q, const GenSrc& k,
-                          const GenSrc& v, float* out, float* part_acc, float* part_ml, size_t part_rows) {
+hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, const DecodeWorkspace* ws, const GenSrc& q,
+                          const GenSrc& k, const GenSrc& v, float* out) {
     const int hd = ctx->head_dim;
+    const bool decode = ws != nullptr;
+    const size_t part_rows = decode ? (size_t)ws->max_splits * ctx->n_heads : ctx->pf_rows;
     const bool norm = ctx->has_qk_norm[layer] != 0;
     GenMmaArgs a;
     a.q = q;
@@ -637,8 +639,6 @@ hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, bool de
     a.kc = ctx->key_cache + (size_t)layer * ctx->layer_elems;
     a.vc = ctx->val_cache + (size_t)layer * ctx->layer_elems;
     a.out = out;
-    a.part_acc = part_acc;
-    a.part_ml = part_ml;
     a.start = start;
     a.n_tok = n_tok;
     a.nh = ctx->n_heads;
@@ -663,6 +663,14 @@ hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, bool de
     ranges = std::min<long long>(ranges, kGmMaxRanges);
     const size_t orows = (size_t)n_tok * a.nh;
     ranges = std::max<long long>(1, std::min<long long>(ranges, (long long)(part_rows / orows)));
+    float *part_acc = nullptr, *part_ml = nullptr;
+    if (ranges > 1) {
+        part_acc = decode ? ws->part_acc : range_partials(ctx, layer);
+        if (part_acc) part_ml = decode ? ws->part_ml : part_acc + part_rows * hd;
+        else ranges = 1;
+    }
+    a.part_acc = part_acc;
+    a.part_ml = part_ml;
     a.nrange = (int)ranges;
     const long long grid = wgs * ranges;
     if (grid > 0x7FFFFFFF || orows > 0x7FFFFFFF) return hipErrorInvalidValue;

@@ -63,9 +63,11 @@ struct pqa_ctx {
     int cu_count = 256;
 
     // prefill partials of key ranges: [pf_rows][head_dim] floats, then
-    // [pf_rows][2]; made with the context, so that a prefill allocates nothing
-    // and captured launches keep a valid address
+    // [pf_rows][2]. pf_part, made with the context, serves the calls that run on
+    // its stream; captured ones, which may be replayed on any stream, have one per
+    // layer (range_partials)
     float* pf_part = nullptr;
+    std::vector<float*> pf_captured;
     size_t pf_rows = 0;
 
     // one allocation for the tables and workspaces whose size the context's
@@ -179,6 +181,9 @@ hipError_t launch_gemm_f16x3_nt(const GemmPlan& plan, const _Float16* a, int lda
                                 int ldc, size_t slice_stride, int m, int n, int kh, hipStream_t stream);
 hipError_t launch_prefill(pqa_ctx* ctx, int layer, int start, int n_tok, const float* q,
                           const float* k, const float* v, float* out);
+// Where a prefill of `layer` leaves the partials of its key ranges (pqa_prefill.hip);
+// null if it must not cut them.
+float* range_partials(pqa_ctx* ctx, int layer);
 // y[t * ld + c] = the sum of a GEMM's K slices part[s * stride + t * cols + c] in slice
 // order, c < cols (an even number), t < n_tok
 struct SliceSum {

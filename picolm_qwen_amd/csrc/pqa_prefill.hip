@@ -966,6 +966,30 @@ static int prefill_ranges(int start, int n_tok, int g, int n_kv, int nblk, int c
     return ranges;
 }
 
+// Calls that run now are in order on the context's stream and share pf_part. A
+// captured one may be replayed on any stream, beside those or beside another captured
+// one, so it gets a buffer of its layer's: only calls of one layer are kept in order
+// by what they do (each reads the cache rows that the other writes). Made by the
+// layer's first capture that cuts keys, in the mode that lets the capturing thread
+// allocate, and kept with the context; without the memory the keys stay whole.
+float* range_partials(pqa_ctx* ctx, int layer) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) (void)hipGetLastError();
+    if (st == hipStreamCaptureStatusNone) return ctx->pf_part;
+    if (ctx->pf_captured.empty()) ctx->pf_captured.assign(ctx->n_layers, nullptr);
+    float*& buf = ctx->pf_captured[layer];
+    if (!buf) {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+        if (hipMalloc((void**)&buf, ctx->pf_rows * (ctx->head_dim + 2) * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            buf = nullptr;
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    return buf;
+}
+
 #ifdef PQA_PHASE_STAMPS
 // The stamped build's extra entry points (not in pqa.h), as for decode.
 extern "C" int pqa_prefill_stamps_read(unsigned long long* dst, int n) {
@@ -1081,10 +1105,11 @@ static hipError_t launch_prefill_hd(pqa_ctx* ctx, int layer, int start, int n_to
         a.qbt = ys->bt[0];
     }
     a.n_tok = n_tok;
-    const int ranges = prefill_ranges(start, n_tok, a.g, a.n_kv, a.nblk, ctx->cu_count, ctx->pf_rows);
+    int ranges = prefill_ranges(start, n_tok, a.g, a.n_kv, a.nblk, ctx->cu_count, ctx->pf_rows);
+    a.part = ranges > 1 ? range_partials(ctx, layer) : nullptr;
+    if (ranges > 1 && !a.part) ranges = prefill_ranges(start, n_tok, a.g, a.n_kv, a.nblk, ctx->cu_count, 0);
     a.nrange = std::max(1, ranges);
-    a.part = ctx->pf_part;
-    a.part_ml = ctx->pf_part + ctx->pf_rows * HD;
+    a.part_ml = a.part ? a.part + ctx->pf_rows * HD : nullptr;
     const dim3 grid((ranges ? a.nblk * ranges : (a.nblk + 1) / 2) * ctx->n_kv_heads);
 #define PQA_PF(SQ, RG) \
     hipLaunchKernelGGL((prefill_attn_kernel<HD, SQ, YS, RG>), grid, dim3(kAttnThreads), 0, ctx->stream, a)

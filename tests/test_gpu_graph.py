@@ -2,7 +2,7 @@
 replayed: every replay, with eager work and synchronisations of the program
 between replays, gives pqa_decode's outputs bit for bit, for one-launch
 per-column steps, split + merge steps and whole-row workgroups; and pqa_prefill
-(which allocates nothing) the same way."""
+the same way."""
 import ctypes as C
 
 import numpy as np
@@ -161,4 +161,80 @@ def test_shorter_prompt_after_a_longer_one_needs_no_new_workspace():
                 assert torch.equal(run[2].view(torch.int32), run[4].view(torch.int32)), (exact_kv, run[0], rep)
         for run in runs:
             run[3].close()
+    att.close()
+
+
+class _KernelNodeParams(C.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint32 * 3),
+                ("args", C.POINTER(C.c_void_p)), ("shared", C.c_uint32)]
+
+
+def _last_kernel_first_pointer(g):
+    """The first argument of the last kernel of a captured chain: the partials that the merge of key
+    ranges reads."""
+    hip = C.CDLL("libamdhip64.so.7")
+    n = C.c_size_t()
+    assert hip.hipGraphGetNodes(g.graph, None, C.byref(n)) == 0
+    nodes = (C.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(g.graph, nodes, C.byref(n)) == 0
+    last = []
+    for node in nodes:
+        deg = C.c_size_t()
+        assert hip.hipGraphNodeGetDependentNodes(C.c_void_p(node), None, C.byref(deg)) == 0
+        if deg.value == 0:
+            last.append(node)
+    assert len(last) == 1 and n.value == 3, (len(last), n.value)  # K/V rows, attention, merge
+    p = _KernelNodeParams()
+    assert hip.hipGraphKernelNodeGetParams(C.c_void_p(last[0]), C.byref(p)) == 0
+    return C.cast(p.args[0], C.POINTER(C.c_void_p))[0]
+
+
+@pytest.mark.parametrize("nh,nkv,hd,start,n", [(8, 2, 128, 3000, 40), (8, 2, 64, 3000, 33), (8, 2, 96, 3000, 40)])
+def test_captured_prompts_of_two_layers_replayed_at_once(nh, nkv, hd, start, n):
+    # prompts whose keys are cut into ranges, captured per layer without an earlier call and replayed on
+    # two streams at once, with an eager one of a third layer on the context's stream: each has partials
+    # of its own, and every result equals the eager call's
+    print(f"graphs at once, {n} tokens at {start}, head size {hd}", flush=True)
+    seed = 9400 + hd
+    cos, sin = O.rope_table(1e6, hd, start + n)
+    att = PicoAttention(3, start + n, nh, nkv, hd, 0, rope_cos=cos, rope_sin=sin)
+    L = _lib.lib()
+    ins, got = [], [torch.zeros(n, nh * hd, device=DEV) for _ in range(3)]
+    for layer in range(3):
+        att.synth_kv(layer, 0, start, seed + layer, 0.01)
+        ins.append([torch.from_numpy(x).to(DEV) for x in O.batch_inputs(seed, layer, 0, n, nh, nkv, hd)])
+    torch.cuda.synchronize()
+
+    def call(layer):
+        q, k, v = ins[layer]
+        assert L.pqa_prefill(att.handle, layer, start, n, _ptr(q), _ptr(k), _ptr(v), _ptr(got[layer])) == 0, att.last_error()
+
+    stream = L.pqa_stream(att.handle)
+    graphs = [Graph(stream, lambda layer=layer: call(layer)) for layer in range(2)]
+    parts = [_last_kernel_first_pointer(g) for g in graphs]
+    assert parts[0] and parts[1] and parts[0] != parts[1]
+    again = Graph(stream, lambda: call(0))  # a layer's later captures use its buffer
+    assert _last_kernel_first_pointer(again) == parts[0]
+    again.close()
+    want = []
+    for layer in range(3):
+        call(layer)
+        att.sync()
+        want.append(got[layer].clone())
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for rep in range(5):
+        for t in got:
+            t.zero_()
+        torch.cuda.synchronize()
+        for _ in range(10):
+            for g, s in zip(graphs, streams):
+                g.launch(s.cuda_stream)
+            call(2)
+        torch.cuda.synchronize()
+        att.sync()
+        for layer in range(3):
+            assert torch.equal(got[layer].view(torch.int32), want[layer].view(torch.int32)), (rep, layer)
+    for g in graphs:
+        g.close()
     att.close()
