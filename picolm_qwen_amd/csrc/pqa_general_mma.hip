@@ -6,10 +6,11 @@
 // The general path computes in fp32, so every operand that is not an fp16 cache
 // value is split into two fp16 parts with 22 significant bits together: q hi + lo
 // (each row first scaled by a power of two so that its largest element lies in
-// [2^14, 2^15)) against K, and P = exp2(score - max + 6) hi + lo against V, both
-// sums in fp32. Rows (query heads of one KV head, token by token) are packed 16 to
-// a wave: S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_f16, in whose
-// layouts a lane's scores are already its operand of the second product. A last
+// [2^14, 2^15)) against K, and P = exp2(score - max + 11) as hi + 2^-11 lo against
+// V, the two parts into sums of their own; all sums in fp32. Rows (query heads of
+// one KV head, token by token) are packed 16 to a wave: S^T = K Q^T and O^T += V^T P^T
+// on v_mfma_f32_16x16x32_f16, in whose layouts a lane's scores are already its
+// operand of the second product. A last
 // half k-step of 16 dims (80, 112) takes v_mfma_f32_16x16x16_f16.
 //
 // K and V tiles of 64 keys (32 in a decode) arrive by direct global->LDS loads, 16-byte chunk c of
@@ -43,8 +44,17 @@
 namespace pqa {
 
 constexpr int kGmRows = 16;    // rows per wave
-constexpr float kGmSlack = 8.0f;  // log2 units between rescales: P stays <= 2^(8 + 6)
-constexpr float kGmShift = 6.0f;  // P is scaled by 2^6: its low part stays clear of fp16 subnormals
+// P = exp2(score - max + kGmShift), rescaled when a score passes the maximum by more
+// than kGmSlack log2 units: at most 2^15, within fp16. Its low part is scaled by kGmLo
+// to the exponents of the high part, and so needs sums of its own: unscaled, both parts
+// end at fp16's 2^-24, and of a key at 2^-30 of the largest weight nothing is left
+// (2e-4 of an output that many such keys beside an attention sink make up; now 3e-8,
+// as with fp32 weights). 22 bits hold down to 2^-25 of the largest weight and 16 at
+// 2^-31, where a score's own fp32 step is 2^-19. The second sums cost 3-4 % of a
+// prefill (up to 7 % at head size 256) and 0.1-0.8 us of a decode.
+constexpr float kGmSlack = 4.0f;
+constexpr float kGmShift = 15.0f - kGmSlack;
+constexpr float kGmLo = 2048.0f;
 
 struct GenMmaArgs {
     GenSrc q, k, v;
@@ -382,9 +392,9 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
     const int qmin = a.start + min(R0, rlast) / a.g;                   // of the wave's first row
     const int qmax = R0 <= rlast ? a.start + min(R0 + kGmRows - 1, rlast) / a.g : -1;
     float m_run = -1e30f, l_run = 0.0f;
-    floatx4 o[DB];  // O^T: dims 16 db + 4 g16 .. +3 of row c16
+    floatx4 o[DB], ol[DB];  // O^T: dims 16 db + 4 g16 .. +3 of row c16; from the high and the low parts of P
 #pragma unroll
-    for (int db = 0; db < DB; db++) o[db] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int db = 0; db < DB; db++) o[db] = ol[db] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto compute = [&](int kt, int buf) __attribute__((always_inline)) {
         const int key0 = kt * KEYS;
@@ -445,8 +455,13 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
             const float corr = fast_exp2(m_run - m_new);
             m_run = m_new;
             l_run *= corr;
+            if (kt > tile0) {  // the first tile has nothing to rescale
 #pragma unroll
-            for (int db = 0; db < DB; db++) o[db] *= corr;
+                for (int db = 0; db < DB; db++) {
+                    o[db] *= corr;
+                    ol[db] *= corr;
+                }
+            }
         }
         const float mref = m_run - kGmShift;
         // k-step h: keys 4 g16 .. +3 of key block 2 h, then of block 2 h + 1
@@ -459,7 +474,7 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
                 l_run += p;
                 const _Float16 hi = (_Float16)p;
                 ph[kb >> 1][4 * (kb & 1) + e] = hi;
-                pl[kb >> 1][4 * (kb & 1) + e] = (_Float16)(p - (float)hi);
+                pl[kb >> 1][4 * (kb & 1) + e] = (_Float16)((p - (float)hi) * kGmLo);
             }
 #pragma unroll
         for (int h = 0; h < KB / 2; h++)
@@ -473,7 +488,7 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
                 const half8 vf = {part[0][0], part[0][1], part[0][2], part[0][3],
                                   part[1][0], part[1][1], part[1][2], part[1][3]};
                 o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[h], o[db], 0, 0, 0);
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[h], o[db], 0, 0, 0);
+                ol[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[h], ol[db], 0, 0, 0);
             }
     };
 
@@ -502,7 +517,10 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
 #pragma unroll
     for (int db = 0; db < DB; db++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) chk = fmaf(o[db][e], 0.0f, chk);
+        for (int e = 0; e < 4; e++) {
+            o[db][e] = fmaf(ol[db][e], 1.0f / kGmLo, o[db][e]);
+            chk = fmaf(o[db][e], 0.0f, chk);
+        }
     const unsigned long long badl = __ballot(!(chk == 0.0f) && R0 + c16 <= rlast);
     const unsigned bad = (unsigned)((badl | badl >> 16 | badl >> 32 | badl >> 48) & 0xFFFFu);
     if (!((bad >> c16) & 1u)) {

@@ -237,3 +237,46 @@ def test_general_mma_host_decode(hd):
     assert_bits_equal(_bits(out), _bits(dev), "host against device entry")
     _check_gen(att, O.shape(nh, nkv, hd, pos + 1, 0), pos, [0], out[None], q, k, v, qn, kn, cos, sin, kc, vc)
     att.close()
+
+
+# many small weights beside one large one (an attention sink with a small V row): what the other keys add is
+# then the whole output, at weights of 2^-31 to 2^-24 or 2^-30 of the largest; matrix-core sizes and VALU ones (72, 100)
+@pytest.mark.parametrize("span", [7.0, 1.0])
+@pytest.mark.parametrize("n_tok", [0, 20])  # 0: a decode
+@pytest.mark.parametrize("hd", [72, 80, 96, 100, 112, 160, 192, 256])
+def test_general_small_weights_beside_a_sink(hd, n_tok, span):
+    print(f"general path, weights 2^-31 to 2^-{31 - span:g} beside a sink, hd {hd}, {n_tok} tokens", flush=True)
+    rng = np.random.default_rng(5500 + hd)
+    nh, nkv, start, n = 4, 1, 3000, max(1, n_tok)
+    smax = start + n
+    cos, sin = np.ones((smax, hd // 2), np.float32), np.zeros((smax, hd // 2), np.float32)  # no rotation
+    att = PicoAttention(1, smax, nh, nkv, hd, 0, rope_cos=cos, rope_sin=sin)
+    unit = np.sqrt(hd) / 1.4426950408889634  # a product of q and k that is one log2 unit of score
+    k = np.zeros((smax, hd), np.float32)
+    k[:, 1] = rng.uniform(0, span, smax) * unit
+    k[0, 0], k[0, 1] = 31 * unit / 8, 0
+    v = rng.standard_normal((smax, hd)).astype(np.float32)
+    v[0] = 0
+    q = np.zeros((n, nh, hd), np.float32)
+    q[..., 0], q[..., 1] = 8, 1
+    q = q.reshape(n, -1)
+    kc, vc = (m[:start].astype(np.float16).view(np.uint16) for m in (k, v))
+    att.kv_upload(0, 0, kc, vc)
+    kc, vc = (np.concatenate([m, np.zeros((n, hd), np.uint16)]) for m in (kc, vc))
+    args = [torch.from_numpy(np.ascontiguousarray(x)).to(DEV) for x in (q, k[start:], v[start:])]
+    if n_tok:
+        out = att.forward_batch(0, start, *args).cpu().numpy()
+    else:
+        out = att.forward(0, start, *(x[0].contiguous() for x in args)).cpu().numpy()[None]
+    shp = O.shape(nh, nkv, hd, smax, 0)
+    for t in range(n):
+        qr = O.append(shp, start + t, q[t], k[start + t], v[start + t], None, None, cos[0], sin[0], kc, vc)
+        want = O.attend_f64(shp, start + t, qr, kc, vc)
+        mag = O.attend_f64(shp, start + t, qr, kc, vc & 0x7FFF)
+        # a score of 31 log2 units has an fp32 step of 2^-19, q 22 bits: 2^-18 of a weight, and as much again for
+        # the weight itself
+        err = np.sqrt(np.mean((out[t] - want) ** 2)) / np.sqrt(np.mean(mag ** 2))
+        if t in (0, n - 1):
+            print(f"  token {t}: {err:.2e} of sum p |v|", flush=True)
+        assert err <= 2.0 ** -17, t
+    att.close()
