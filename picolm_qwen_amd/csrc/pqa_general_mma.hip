@@ -35,8 +35,8 @@
 //
 // Infinities: a split product can turn inf into NaN (inf * 0, inf - inf), and a
 // masked key's V row still enters the product with weight 0. A row whose result is
-// not finite is therefore computed again by gen_row, with fp32 q, only its own
-// keys and no split.
+// not finite is therefore computed again by gen_rows, with fp32 q and P, only its
+// own keys and no split.
 #include <algorithm>
 
 #include "pqa_general.h"
@@ -102,61 +102,132 @@ __device__ __forceinline__ float4 gm_load4(const GenSrc& s, int t, int c, int ve
     return *(const float4*)(s.p + (size_t)t * s.ld + c);
 }
 
-// The row at q (fp32, prepared) over the keys of tiles first, first + step, ...
-// below end that are at most qpos, in fp32: m, l and the accumulator (row acc, may
-// alias q) in the scale of the MFMA path. One wave.
+// Four of a wave's rows again, rows row0 .. row0 + 3 of which those in `bad`: the rows
+// at q (fp32, prepared), each over its own keys of tiles first, first + step, ... below
+// end, in fp32. Row, m and l of each go to res, m_out and l_out in the
+// scale of the MFMA path (res may alias q). Lane = key for the scores (64 keys at a
+// time), lane = pair of dims for the sums over V, whose rows come 16 or 32 at a time,
+// ahead of the sums over those before; four rows share each K and V load. With an infinite V row in the cache (every row of a
+// wave again), per layer, the VALU kernels' time in brackets: 700 tokens of 32 / 8
+// heads of 96 270 us (210), 32 / 32 of 80 267 (340), 8 / 2 of 256 710 (272: 88
+// workgroups); decode at 9000 keys 21 (33), 55 (46) and 32 us (46). One row after the
+// other, each with K and V loads of its own, took 2460, 2390, 1900, 67, 157 and 38.
 template <int HD, int KEYS>
-__device__ void gen_row(const uint16_t* kbase, const uint16_t* vbase, size_t stride, const float* q, int qpos, int first,
-                        int step, int end, int lane, float* acc_row, float& m_out, float& l_out) {
-    constexpr int NA = (HD + 63) / 64;
-    float m = -1e30f, l = 0.0f, acc[NA];
+__device__ __forceinline__ void gen_rows(const GenMmaArgs& a, const uint16_t* kbase, const uint16_t* vbase, const float* q,
+                                         int row0, unsigned bad, int first, int step, int end, int lane, float* res,
+                                         float* m_out, float* l_out) {
+    constexpr int QS = HD + 4, NP = (HD / 2 + 63) / 64;  // LDS row stride; dim pairs per lane
+    constexpr int TPI = 64 / KEYS;                       // tiles at a time
+    constexpr int VB = 32 / NP;                          // V rows at a time
+    const size_t stride = (size_t)a.kv_dim;
+    int qp[4];
 #pragma unroll
-    for (int i = 0; i < NA; i++) acc[i] = 0.0f;
-    for (int kt = first; kt < end; kt += step) {
-        const int key0 = kt * KEYS, nk = min(KEYS, qpos + 1 - key0);
-        if (nk <= 0) break;
-        const bool valid = lane < nk;
-        const u32x4* kr = (const u32x4*)(kbase + (size_t)(key0 + (valid ? lane : 0)) * stride);
-        float s = 0.0f;
+    for (int r = 0; r < 4; r++) qp[r] = a.start + min(row0 + r, a.rows - 1) / a.g;
+    const int qlast = qp[3];
+    float m[4], l[4], acc[4][2 * NP];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        m[r] = -1e30f;
+        l[r] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 2 * NP; i++) acc[r][i] = 0.0f;
+    }
+    // the first key of batch b of V rows, of tiles kt, kt + step; past qlast: nothing
+    auto batch_key = [&](int kt, int b) __attribute__((always_inline)) {
+        const int tile = kt + VB * b / KEYS * step;
+        return tile < end ? tile * KEYS + VB * b % KEYS : qlast + 1;
+    };
+    auto load_v = [&](int kt, int b, uint32_t (&v)[VB][NP]) __attribute__((always_inline)) {
+        const int key0 = batch_key(kt, b);
+        if (key0 > qlast) return;
+#pragma unroll
+        for (int u = 0; u < VB; u++) {
+            const uint16_t* vr = vbase + (size_t)min(key0 + u, qlast) * stride;
+#pragma unroll
+            for (int i = 0; i < NP; i++) v[u][i] = 2 * (lane + 64 * i) < HD ? *(const uint32_t*)(vr + 2 * (lane + 64 * i)) : 0u;
+        }
+    };
+    auto add_v = [&](int kt, int b, const uint32_t (&v)[VB][NP], const float (&p)[4]) __attribute__((always_inline)) {
+        const int key0 = batch_key(kt, b);
+        if (key0 > qlast) return;
+        auto add = [&](int u, int r) __attribute__((always_inline)) {
+            const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[r]), VB * b + u));
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                acc[r][2 * i] = fmaf(pj, f16_bits_to_f32((uint16_t)(v[u][i] & 0xFFFFu)), acc[r][2 * i]);
+                acc[r][2 * i + 1] = fmaf(pj, f16_bits_to_f32((uint16_t)(v[u][i] >> 16)), acc[r][2 * i + 1]);
+            }
+        };
+        if (key0 + VB - 1 <= qp[0]) {  // every key is every row's
+#pragma unroll
+            for (int u = 0; u < VB; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) add(u, r);
+        } else {
+#pragma unroll
+            for (int u = 0; u < VB; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (key0 + u <= qp[r]) add(u, r);
+        }
+    };
+    for (int kt = first; kt < end && kt * KEYS <= qlast; kt += TPI * step) {
+        uint32_t v[2][VB][NP];
+        load_v(kt, 0, v[0]);
+        const int tile = kt + lane / KEYS * step, key = tile * KEYS + lane % KEYS;
+        const bool in = tile < end && key <= qlast;
+        const u32x4* kr = (const u32x4*)(kbase + (size_t)(in ? key : kt * KEYS) * stride);
+        float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
         for (int c = 0; c < HD / 8; c++) {
             const u32x4 u = kr[c];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                s = fmaf(q[8 * c + 2 * e], f16_bits_to_f32((uint16_t)(u[e] & 0xFFFFu)), s);
-                s = fmaf(q[8 * c + 2 * e + 1], f16_bits_to_f32((uint16_t)(u[e] >> 16)), s);
+            for (int r = 0; r < 4; r++) {
+                const float* x = q + r * QS + 8 * c;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    s[r] = fmaf(x[2 * e], f16_bits_to_f32((uint16_t)(u[e] & 0xFFFFu)), s[r]);
+                    s[r] = fmaf(x[2 * e + 1], f16_bits_to_f32((uint16_t)(u[e] >> 16)), s[r]);
+                }
             }
         }
-        const float sv = valid ? s : -__builtin_huge_valf();
-        const float mn = fmaxf(m, group_max<64>(sv));
-        const float corr = fast_exp2(m - mn);
-        const float p = valid ? fast_exp2(sv - mn + kGmShift) : 0.0f;
-        l = l * corr + group_sum<64>(p);
-        m = mn;
+        float p[4];
 #pragma unroll
-        for (int i = 0; i < NA; i++) acc[i] *= corr;
-        for (int j = 0; j < nk; j++) {
-            const float pj = __shfl(p, j);
-            const uint16_t* vr = vbase + (size_t)(key0 + j) * stride;
+        for (int r = 0; r < 4; r++) {
+            const bool valid = in && key <= qp[r];
+            const float sv = valid ? s[r] : -__builtin_huge_valf();
+            const float mn = fmaxf(m[r], group_max<64>(sv));
+            const float corr = fast_exp2(m[r] - mn);
+            p[r] = valid ? fast_exp2(sv - mn + kGmShift) : 0.0f;
+            l[r] = l[r] * corr + group_sum<64>(p[r]);
+            m[r] = mn;
 #pragma unroll
-            for (int i = 0; i < NA; i++) {
-                const int d = lane + 64 * i;
-                if (d < HD) acc[i] = fmaf(pj, f16_bits_to_f32(vr[d]), acc[i]);
-            }
+            for (int i = 0; i < 2 * NP; i++) acc[r][i] *= corr;
+        }
+#pragma unroll
+        for (int b = 0; b < 64 / VB; b++) {
+            if (b + 1 < 64 / VB) load_v(kt, b + 1, v[(b + 1) & 1]);
+            add_v(kt, b, v[b & 1], p);
         }
     }
     wave_sync();  // q has been read
 #pragma unroll
-    for (int i = 0; i < NA; i++)
-        if (lane + 64 * i < HD) acc_row[lane + 64 * i] = acc[i];
-    wave_sync();
-    m_out = m;
-    l_out = l;
+    for (int r = 0; r < 4; r++) {
+        if (!((bad >> r) & 1u)) continue;
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+            if (2 * (lane + 64 * i) < HD) *(float2*)(res + r * QS + 2 * (lane + 64 * i)) = float2{acc[r][2 * i], acc[r][2 * i + 1]};
+        if (lane == 0) {
+            m_out[r] = m[r];
+            l_out[r] = l[r];
+        }
+    }
 }
 
 // DECODE: one row group (16 query heads of one KV head at one token), waves on
 // different key tiles; else 4 row groups on the same tiles.
 template <int HD, bool DECODE>
-__global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen_mma_kernel(const GenMmaArgs a) {
+__global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256, !DECODE && HD <= 96 ? 2 : 1) void gen_mma_kernel(const GenMmaArgs a) {
     constexpr int KEYS = gm_keys<HD, DECODE>(), KB = KEYS / 16;
     using T = GmTile<HD, KEYS>;
     constexpr int NW = DECODE ? gm_decode_waves<HD>() : 4;
@@ -534,15 +605,11 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256) void gen
     wave_sync();
     if (bad) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the new row's stores
-        for (int r = 0; r < kGmRows; r++) {
-            if (!((bad >> r) & 1u)) continue;
-            float mr, lr;
-            gen_row<HD, KEYS>((const uint16_t*)kbase, (const uint16_t*)vbase, (size_t)a.kv_dim, qreg + r * QS,
-                        a.start + (R0 + r) / a.g, tile0, KW, tile1, lane, res + r * QS, mr, lr);
-            if (lane == 0) {
-                s_ml[w][0][r] = mr;
-                s_ml[w][1][r] = lr;
-            }
+#pragma unroll 1
+        for (int r = 0; r < kGmRows; r += 4) {
+            if (!((bad >> r) & 15u)) continue;
+            gen_rows<HD, KEYS>(a, (const uint16_t*)kbase, (const uint16_t*)vbase, qreg + r * QS, R0 + r, bad >> r, tile0, KW,
+                               tile1, lane, res + r * QS, &s_ml[w][0][r], &s_ml[w][1][r]);
         }
         wave_sync();
     }

@@ -280,3 +280,45 @@ def test_general_small_weights_beside_a_sink(hd, n_tok, span):
             print(f"  token {t}: {err:.2e} of sum p |v|", flush=True)
         assert err <= 2.0 ** -17, t
     att.close()
+
+
+# the same rows among several key ranges (decode: several waves and workgroups; prefill: blocks cut in two or
+# more), with infinite and NaN rows in the first, a middle and the last range, the new rows among them; groups of
+# rows at one position and at sixteen
+@pytest.mark.parametrize("hd,nh,nkv", [(80, 4, 4), (96, 8, 2), (112, 17, 1), (160, 4, 1), (192, 2, 2), (256, 8, 2)])
+def test_general_mma_non_finite_rows_in_ranges(hd, nh, nkv):
+    print(f"general path, infinite cache rows in several ranges, {nh}/{nkv} x {hd}", flush=True)
+    start, n_tok, seed, kvd = 2100, 40, 5600 + hd, nkv * hd
+    smax = start + n_tok
+    cos, sin = np.ones((smax, hd // 2), np.float32), np.zeros((smax, hd // 2), np.float32)  # no rotation
+    att = PicoAttention(1, smax, nh, nkv, hd, 0, rope_cos=cos, rope_sin=sin)
+    kc, vc = np.zeros((smax, kvd), np.uint16), np.zeros((smax, kvd), np.uint16)
+    kc[:start], vc[:start] = O.synth_kv_rows(seed, 0, kvd, 0, start, 0.0)
+    inf, ninf = 0x7C00, 0xFC00
+    kc[[5, 1000, 2090], 0::hd] = ninf  # dim 0 of q is positive: score -inf, weight 0
+    vc[3, 4], vc[3, 9] = inf, 0x7E00   # infinite and NaN in every output
+    vc[1111, 6] = ninf
+    vc[2095, 8] = inf
+    q, k, v = (x.copy() for x in O.batch_inputs(seed, 0, 0, n_tok, nh, nkv, hd))
+    q[:, 0::hd] = np.abs(q[:, 0::hd]) + 0.1
+    k[7, 0] = -1e6
+    v[20, 10] = 1e6   # dim 10 infinite from token 20 on
+    v[33, 12] = -1e6  # and a new token whose own row is infinite
+    v[33, 6] = 1e6    # +inf after -inf: NaN from token 33 on
+    att.kv_upload(0, 0, kc[:start], vc[:start])
+    dq, dk, dv = (torch.from_numpy(x).to(DEV) for x in (q, k, v))
+    out = att.forward_batch(0, start, dq, dk, dv).cpu().numpy()
+    shp = O.shape(nh, nkv, hd, smax, 0)
+    dec = {}
+    for t in (0, 19, 20, 33, n_tok - 1):  # the decode of a token, over the rows the prompt left before it
+        dec[t] = att.forward(0, start + t, dq[t].contiguous(), dk[t].contiguous(), dv[t].contiguous()).cpu().numpy()
+    for t in range(n_tok):
+        qr = O.append(shp, start + t, q[t], k[t], v[t], None, None, cos[0], sin[0], kc, vc)
+        want = O.attend(shp, start + t, qr, kc, vc)
+        assert np.isfinite(want).any() and np.isinf(want).any() and np.isnan(want).any()
+        for got in [out[t]] + ([dec[t]] if t in dec else []):
+            assert np.array_equal(np.isnan(got), np.isnan(want)), t
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]), t
+            fin = np.isfinite(want)
+            assert np.all(np.abs(got[fin] - want[fin]) <= 1e-4), t
+    att.close()
