@@ -411,7 +411,7 @@ static int ensure_layer_exact(pqa_ctx* ctx, int layer, const char* fn) {
     const int n = p.n_embd, rows = (int)ctx->kv_dim;
     const size_t fk = pqa::exact_matrix_floats(p.wtype[1], rows, n);
     const size_t fv = pqa::exact_matrix_floats(p.wtype[2], rows, n);
-    if (int rc = ensure_batch(ctx, (size_t)rows * n, fn)) return rc;
+    if (int rc = ensure_batch(ctx, ctx->q_dim * (size_t)n, fn)) return rc;  // what the layer's split weights take
     float* buf = nullptr;
     if (int rc = hip_check(ctx, hipMalloc(&buf, (fk + fv) * 4), fn)) return rc;
     hipError_t e = pqa::prepare_exact_matrix(p.wtype[1], p.w[1], p.stride[1], rows, n, ctx->wf32, buf, ctx->stream);
