@@ -39,3 +39,22 @@ def make_rows(rng, wtype, rows, n, special=False):
 def make_bias(rng, btype, rows):
     b = (rng.standard_normal(rows) * 0.1)
     return b.astype("<f4").view(np.uint8) if btype == O.GGUF_F32 else b.astype("<f2").view(np.uint8)
+
+
+# shapes for the split GEMM of the batched projections: tokens, input width, query heads of 64 (one KV head), output
+# rows, and the plan (tile mi, nj and K slices on 256 CUs) of the q, the q/k/v and the output product. Every tile, with
+# and without slices (64 x 64 up to 256 x 192); partial tiles; K of one, an odd number and many 32-wide steps.
+GEMM_CASES = [
+    (1, 8, 3, 32, (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+    (63, 40, 3, 160, (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+    (65, 1000, 3, 4000, (1, 1, 16), (1, 1, 16), (1, 1, 1)),
+    (128, 2048, 16, 8192, (1, 1, 8), (1, 1, 7), (1, 1, 1)),
+    (129, 896, 14, 3584, (1, 1, 6), (1, 1, 5), (1, 1, 1)),
+    (257, 1032, 32, 4128, (1, 1, 1), (1, 1, 1), (2, 1, 1)),
+    (513, 2560, 32, 10240, (2, 2, 3), (2, 2, 3), (4, 2, 1)),
+    (1025, 512, 44, 2048, (2, 2, 1), (2, 2, 1), (4, 2, 3)),
+    (75, 2560, 64, 2560, (2, 1, 4), (2, 1, 3), (2, 1, 6)),
+    (2047, 160, 96, 160, (4, 3, 1), (4, 2, 1), (2, 1, 5)),
+    (700, 2560, 96, 2560, (4, 3, 2), (4, 3, 2), (2, 1, 1)),
+    (1999, 128, 64, 2560, (4, 2, 1), (4, 3, 1), (4, 3, 2)),
+]

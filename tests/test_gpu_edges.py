@@ -6,7 +6,7 @@ import pytest
 
 import oracle as O
 from gpu_util import assert_bits_equal
-from proj_cases import make_bias, make_rows
+from proj_cases import GEMM_CASES, make_bias, make_rows
 
 torch = pytest.importorskip("torch")
 from picolm_qwen_amd import PicoAttention  # noqa: E402
@@ -44,13 +44,51 @@ def test_ordered_projection_tile_edges(n_tok, kt, vt, dim):
     att.close()
 
 
-# the split GEMM's workgroup tiles (64 to 256 rows, 64 to 192 columns, with and without K
-# slices): token counts around the tile edges, widths whose K is one, an odd number and many
-# 32-wide tiles, and columns that leave partial tiles
-@pytest.mark.parametrize("n_tok,dim,nh", [(1, 8, 3), (63, 40, 3), (65, 1000, 3), (128, 2048, 16), (129, 896, 14),
-                                          (257, 1032, 32), (513, 2560, 32), (1025, 512, 44)])
-def test_split_gemm_tile_edges(n_tok, dim, nh):
-    print(f"split GEMM, {n_tok} tokens, width {dim}, {nh} heads", flush=True)
+# infinities, NaN, subnormals, zeros of both signs and products that overflow or vanish, in weights and
+# inputs: every K and V element is the oracle's bits, or NaN where its is NaN
+@pytest.mark.parametrize("n_tok", [3, 300])  # 16 x 16 and 32 x 32 tiles
+@pytest.mark.parametrize("kt", [O.GGUF_F32, O.GGUF_F16, O.GGUF_Q8_0])
+def test_ordered_projection_special_values(kt, n_tok):
+    print(f"reference-order K/V of special values, type {kt}, {n_tok} tokens", flush=True)
+    rng = np.random.default_rng(900 + kt + n_tok)
+    nkv, hd, dim = 8, 128, 320
+    att = PicoAttention(1, 16, nkv, nkv, hd)
+    rows = nkv * hd
+    w = [make_rows(rng, kt, rows, dim, special=True) for _ in range(3)]
+    special = np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, 1e-45, -1e-40, 1.2e-38, 3e38, -3e38, 2e-23], np.float32)
+    x = rng.standard_normal((n_tok, dim)).astype(np.float32)
+    x[rng.random(x.shape) < 0.3] *= np.float32(1e-38)
+    at = rng.random(x.shape) < 0.3
+    x[at] = rng.choice(special[3:], at.sum()) / (1 if kt == O.GGUF_F32 else 2048)  # int8 and fp16 weights are larger
+    for t in range(0, n_tok, 3):  # a third of the tokens, so that most sums stay finite
+        x[t, 11], x[t, 200] = np.inf, special[t // 3 % 3]
+    x[-1] = rng.standard_normal(dim)
+    for m in w:
+        if kt == O.GGUF_Q8_0:
+            m.reshape(rows, dim // 32, 34)[::7, 3, :2] = np.array([0x7C00], "<u2").view(np.uint8)  # infinite scales
+            continue
+        f = m.view("<f4" if kt == O.GGUF_F32 else "<f2").reshape(rows, dim)
+        finite = special[3:] if kt == O.GGUF_F32 else np.array([0.0, -0.0, 6e-8, -3e-6, 6.2e-5, 65504, -65504], np.float32)
+        at = rng.random(f.shape) < 0.2
+        f[at] = rng.choice(finite, at.sum())
+        f[::5, 17] = rng.choice(np.concatenate([special[:3], finite]), rows // 5 + 1)
+    att.set_qkv_weights(0, dim, w[0], kt, w[1], kt, w[2], kt)
+    _, k, v = (g.cpu().numpy() for g in att.qkv_project_batch(0, torch.from_numpy(x).to(DEV)))
+    for name, g, m in (("k", k, w[1]), ("v", v, w[2])):
+        want = O.matmul_bias_tokens(x, m, kt, rows)
+        nan = np.isnan(want)
+        assert 0.01 < nan.mean() < 0.9 and np.isinf(want).any()
+        assert np.array_equal(np.isnan(g), nan), name
+        assert_bits_equal(_bits(np.where(nan, 0, g)), _bits(np.where(nan, 0, want)), name)
+    att.close()
+
+
+# the split GEMM's workgroup tiles (64 to 256 rows, 64 to 192 columns, each with and without K
+# slices): the shapes of GEMM_CASES, whose plans a CPU test checks
+@pytest.mark.parametrize("n_tok,dim,nh,out_rows", [c[:4] for c in GEMM_CASES])
+def test_split_gemm_tile_edges(n_tok, dim, nh, out_rows):
+    print(f"split GEMM, {n_tok} tokens, width {dim}, {nh} heads, {out_rows} output rows", flush=True)
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256  # what the plans are for
     rng = np.random.default_rng(7 * n_tok + dim)
     nkv, hd, wt = 1, 64, O.GGUF_F32
     att = PicoAttention(1, 16, nh, nkv, hd)
@@ -58,37 +96,52 @@ def test_split_gemm_tile_edges(n_tok, dim, nh):
     w = [make_rows(rng, wt, r, dim) for r in rows]
     b = make_bias(rng, O.GGUF_F32, rows[0])
     att.set_qkv_weights(0, dim, w[0], wt, w[1], wt, w[2], wt, b, O.GGUF_F32)
-    wo, bo = make_rows(rng, wt, 4 * dim, nh * hd), make_bias(rng, O.GGUF_F32, 4 * dim)
-    att.set_out_weights(0, 4 * dim, wo, wt, bo, O.GGUF_F32)
-    x = rng.standard_normal((n_tok, dim)).astype(np.float32)
+    wo, bo = make_rows(rng, wt, out_rows, nh * hd), make_bias(rng, O.GGUF_F32, out_rows)
+    att.set_out_weights(0, out_rows, wo, wt, bo, O.GGUF_F32)
     wf = [m.view(np.float32).astype(np.float64) for m in (*w, wo)]
-    # 3 n products of 22-bit operands: within (3 n + 12) 2^-24 sum |w x| of the exact sum, and a
-    # rounding of the bias sum (and of the residual sum) on top
+    # every token of a small prompt, the edges of every tile and some within of a large one
+    some = np.arange(n_tok) if n_tok * dim * nh < 1e8 else np.array(
+        sorted({0, 1, n_tok - 1} | {t + d for t in range(64, n_tok, 64) for d in (-1, 0)} | set(range(5, n_tok, 97))))
+
+    def check(got, x, wm, bias, residual, name):
+        x = x[some].astype(np.float64)
+        want = x @ wm.T + bias
+        mag = np.abs(x) @ np.abs(wm).T
+        got = got[some].astype(np.float64)
+        # 3 n products of 22-bit operands: within (3 n + 12) 2^-24 sum |w x| of the exact sum, and a rounding of the
+        # bias sum (and of the residual sum) on top
+        last = 2.0 ** -23 * (np.abs(want) + (np.abs(want + residual) if residual is not None else 0))
+        full = want if residual is None else want + residual
+        err = np.abs(got - full)
+        assert np.all(err <= (3 * wm.shape[1] + 12) * 2.0 ** -24 * mag + last + 1e-30), name
+        # and in the mean square (less that last rounding) far below what a product without a low part would be off,
+        # 2^-13.3 of sqrt(sum w^2 x^2): rounding at 22 bits gives about 2^-22 of it, the fp32 sums 2^-24 sqrt(n)
+        rms = np.sqrt(np.mean(np.maximum(err - last, 0) ** 2))
+        assert rms <= 2.0 ** -17 * np.sqrt(np.mean((x * x) @ (wm * wm).T)), (name, rms)
+
+    x = rng.standard_normal((n_tok, dim)).astype(np.float32)
     for exact_kv in (False, True):
         att.set_batch_projection(exact_kv)
-        got = [g.cpu().numpy().astype(np.float64) for g in att.qkv_project_batch(0, torch.from_numpy(x).to(DEV))]
+        got = [g.cpu().numpy() for g in att.qkv_project_batch(0, torch.from_numpy(x).to(DEV))]
         for j in range(1 if exact_kv else 3):
-            want = x.astype(np.float64) @ wf[j].T + (b.view(np.float32) if j == 0 else 0.0)
-            mag = np.abs(x.astype(np.float64)) @ np.abs(wf[j]).T
-            assert np.all(np.abs(got[j] - want) <= (3 * dim + 12) * 2.0 ** -24 * mag + 2.0 ** -23 * np.abs(want) + 1e-30), j
+            check(got[j], x, wf[j], b.view(np.float32) if j == 0 else 0.0, None, "qkv"[j])
     a = rng.standard_normal((n_tok, nh * hd)).astype(np.float32)
-    x0 = rng.standard_normal((n_tok, 4 * dim)).astype(np.float32)
+    x0 = rng.standard_normal((n_tok, out_rows)).astype(np.float32)
     xo = torch.from_numpy(x0.copy()).to(DEV)
     att.out_project_batch(0, torch.from_numpy(a).to(DEV), xo)
-    y = a.astype(np.float64) @ wf[3].T + bo.view(np.float32)
-    mag = np.abs(a.astype(np.float64)) @ np.abs(wf[3]).T
-    tol = (3 * nh * hd + 12) * 2.0 ** -24 * mag + 2.0 ** -23 * (np.abs(y) + np.abs(y + x0)) + 1e-30
-    assert np.all(np.abs(xo.cpu().numpy() - (y + x0)) <= tol)
+    check(xo.cpu().numpy(), a, wf[3], bo.view(np.float32), x0[some], "out")
     att.close()
 
 
 # prefill behind a history: blocks whose keys are cut into ranges (few blocks, a long history),
-# ranges past a row's own position, one block per workgroup without ranges, and prompts that
-# stay on block pairs; both head sizes, both q precisions
+# ranges past a row's own position and empty ones of the first blocks (a prompt at 0), one block
+# per workgroup without ranges, and prompts that stay on block pairs; both head sizes, both q precisions
 @pytest.mark.parametrize("nh,nkv,hd,start,n_tok,split_q", [(4, 1, 64, 3000, 5, True), (2, 1, 128, 1000, 100, True),
                                                            (7, 1, 64, 700, 65, False), (8, 2, 128, 2047, 1, True),
                                                            (4, 2, 128, 64, 300, True), (32, 2, 64, 129, 700, True),
-                                                           (32, 1, 128, 500, 2100, False)])
+                                                           (32, 1, 128, 500, 2100, False),
+                                                           (2, 1, 128, 0, 2048, True), (8, 2, 128, 3000, 40, False),
+                                                           (4, 1, 64, 0, 1500, False)])
 def test_prefill_key_ranges(nh, nkv, hd, start, n_tok, split_q):
     print(f"prefill ranges {nh}/{nkv} x {hd}, {n_tok} tokens at {start}, split_q {split_q}", flush=True)
     smax, seed, kvd = start + n_tok, 4100 + start, nkv * hd

@@ -29,6 +29,8 @@ DECODE = [
     ("hd48_g12_chunks_pos0", 24, 2, 48, 16, 0, 1e6, True, 0, 0.0),
     ("hd2_pos70", 4, 2, 2, 128, 0, 1e4, False, 70, 0.0),
     ("hd72_long_pos20000", 16, 2, 72, 20480, 0, 1e6, False, 20000, 0.0),
+    ("hd144_qknorm_pos1500", 8, 2, 144, 2048, 0, 1e6, True, 1500, 0.01),
+    ("hd208_g12_chunks_pos65", 24, 2, 208, 128, 1, 1e4, False, 65, 0.0),
 ]
 
 
@@ -76,6 +78,11 @@ PREFILL = [
     ("hd100_block8_tail_start40_n70", 8, 2, 100, 160, 1, 1e4, True, 40, 70),
     ("hd256_neox_start5_n64", 8, 2, 256, 128, 0, 1e6, True, 5, 64),
     ("hd80_interleaved_g12_n33", 24, 2, 80, 64, 2, 1e4, False, 0, 33),
+    # sizes on the VALU kernels whose heads are whole 16-byte chunks, as those above on the matrix cores
+    ("hd72_block8_n150", 16, 4, 72, 256, 1, 1e4, True, 0, 150),
+    ("hd72_interleaved_g12_start300_n33", 24, 2, 72, 400, 2, 1e4, False, 300, 33),
+    ("hd144_neox_start5_n64", 8, 2, 144, 128, 0, 1e6, True, 5, 64),
+    ("hd208_g12_n40", 24, 2, 208, 64, 0, 1e6, False, 0, 40),
 ]
 
 
@@ -126,20 +133,23 @@ def test_general_prefill_row_equals_decode():
     dec.close()
 
 
-def test_general_from_xb_paths():
-    # head_dim 96 with Q8_0 projections: pqa_decode_x (projections bit-exact,
+@pytest.mark.parametrize("exact_kv", [True, False])
+@pytest.mark.parametrize("hd", [96, 72, 144])  # matrix cores, and the VALU kernels' two widths
+def test_general_from_xb_paths(hd, exact_kv):
+    # Q8_0 projections: pqa_decode_x (projections bit-exact,
     # so the appended rows are too) against the oracle, and pqa_prefill_x (the
     # batched GEMM's scaled result read by the general prep kernel) bit-equal
     # to pqa_qkv_project_batch followed by pqa_prefill on a twin context
-    print("general head_dim from xb", flush=True)
-    rng = np.random.default_rng(96)
-    nh, nkv, hd, dim, smax, n_tok = 16, 4, 96, 1024, 128, 50
+    print(f"general head_dim {hd} from xb, exact K/V {exact_kv}", flush=True)
+    rng = np.random.default_rng(hd)
+    nh, nkv, dim, smax, n_tok = 16, 4, 1024, 128, 50
     wt = O.GGUF_Q8_0
     wq, wk, wv = (make_rows(rng, wt, r, dim) for r in (nh * hd, nkv * hd, nkv * hd))
     ctxs = []
     for _ in range(2):
         att, cos, sin, qn, kn = _context(nh, nkv, hd, smax, 0, 1e6, True, 7)
         att.set_qkv_weights(0, dim, wq, wt, wk, wt, wv, wt)
+        att.set_batch_projection(exact_kv)
         ctxs.append(att)
     x = rng.standard_normal((n_tok, dim)).astype(np.float32)
     a = ctxs[0].forward_batch_x(0, 0, torch.from_numpy(x).to(DEV)).cpu().numpy()

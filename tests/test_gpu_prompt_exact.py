@@ -100,7 +100,7 @@ def test_batch_kv_equals_per_token_projection():
 
 
 def test_prefill_x_general_head_dim_rows_exact():
-    # head_dim 96 takes the VALU attention kernels; their K/V prep reads the
+    # head_dim 96 takes the general path's K/V prep, which reads the
     # reference-order columns as they are
     print("prefill_x hd 96, reference-order K/V", flush=True)
     rng = np.random.default_rng(3496)
