@@ -6,7 +6,7 @@
 // The general path computes in fp32, so every operand that is not an fp16 cache
 // value is split into two fp16 parts with 22 significant bits together: q hi + lo
 // (each row first scaled by a power of two so that its largest element lies in
-// [2^14, 2^15)) against K, and P = exp2(score - max + 11) as hi + 2^-11 lo against
+// [2^14, 2^15)) against K, and P = 2^11 exp2(score - max) as hi + 2^-11 lo against
 // V, the two parts into sums of their own; all sums in fp32. Rows (query heads of
 // one KV head, token by token) are packed 16 to a wave: S^T = K Q^T and O^T += V^T P^T
 // on v_mfma_f32_16x16x32_f16, in whose layouts a lane's scores are already its
@@ -44,16 +44,17 @@
 namespace pqa {
 
 constexpr int kGmRows = 16;    // rows per wave
-// P = exp2(score - max + kGmShift), rescaled when a score passes the maximum by more
-// than kGmSlack log2 units: at most 2^15, within fp16. Its low part is scaled by kGmLo
-// to the exponents of the high part, and so needs sums of its own: unscaled, both parts
-// end at fp16's 2^-24, and of a key at 2^-30 of the largest weight nothing is left
-// (2e-4 of an output that many such keys beside an attention sink make up; now 3e-8,
-// as with fp32 weights). 22 bits hold down to 2^-25 of the largest weight and 16 at
-// 2^-31, where a score's own fp32 step is 2^-19. The second sums cost 3-4 % of a
-// prefill (up to 7 % at head size 256) and 0.1-0.8 us of a decode.
+// P = 2^11 exp2(score - max), rescaled when a score passes the maximum by more than
+// kGmSlack log2 units: at most 2^15, within fp16. (The factor is exact; 11 added to the
+// exponent would round it at 2^-21.) Its low part is scaled by kGmLo to the exponents of
+// the high part, and so needs sums of its own: unscaled, both parts end at fp16's 2^-24,
+// and of a key at 2^-30 of the largest weight nothing is left (2e-4 of an output that
+// many such keys beside an attention sink make up; now 3e-8, as with fp32 weights). 22
+// bits hold down to 2^-25 of the largest weight and 16 at 2^-31, where a score's own
+// fp32 step is 2^-19. The second sums cost 3-4 % of a prefill at head size 112 or more
+// (up to 7 % at 256) and 0.1-0.8 us of a decode.
 constexpr float kGmSlack = 4.0f;
-constexpr float kGmShift = 15.0f - kGmSlack;
+constexpr float kGmScale = 2048.0f;
 constexpr float kGmLo = 2048.0f;
 
 struct GenMmaArgs {
@@ -198,7 +199,7 @@ __device__ __forceinline__ void gen_rows(const GenMmaArgs& a, const uint16_t* kb
             const float sv = valid ? s[r] : -__builtin_huge_valf();
             const float mn = fmaxf(m[r], group_max<64>(sv));
             const float corr = fast_exp2(m[r] - mn);
-            p[r] = valid ? fast_exp2(sv - mn + kGmShift) : 0.0f;
+            p[r] = valid ? fast_exp2(sv - mn) * kGmScale : 0.0f;
             l[r] = l[r] * corr + group_sum<64>(p[r]);
             m[r] = mn;
 #pragma unroll
@@ -534,14 +535,13 @@ __global__ __launch_bounds__(DECODE ? 64 * gm_decode_waves<HD>() : 256, !DECODE 
                 }
             }
         }
-        const float mref = m_run - kGmShift;
         // k-step h: keys 4 g16 .. +3 of key block 2 h, then of block 2 h + 1
         half8 ph[KB / 2], pl[KB / 2];
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const float p = fast_exp2(s[kb][e] - mref);
+                const float p = fast_exp2(s[kb][e] - m_run) * kGmScale;
                 l_run += p;
                 const _Float16 hi = (_Float16)p;
                 ph[kb >> 1][4 * (kb & 1) + e] = hi;

@@ -115,7 +115,7 @@ def test_split_gemm_tile_edges(n_tok, dim, nh, out_rows):
         err = np.abs(got - full)
         assert np.all(err <= (3 * wm.shape[1] + 12) * 2.0 ** -24 * mag + last + 1e-30), name
         # and in the mean square (less that last rounding) far below what a product without a low part would be off,
-        # 2^-13.3 of sqrt(sum w^2 x^2): rounding at 22 bits gives about 2^-22 of it, the fp32 sums 2^-24 sqrt(n)
+        # 2^-12.2 of sqrt(sum w^2 x^2): the split gives 2^-23.7 of it, the fp32 sums at most 2^-24 sqrt(3 n)
         rms = np.sqrt(np.mean(np.maximum(err - last, 0) ** 2))
         assert rms <= 2.0 ** -17 * np.sqrt(np.mean((x * x) @ (wm * wm).T)), (name, rms)
 
