@@ -54,10 +54,12 @@ typedef enum {
  * rope_cos/rope_sin: host, [max_seq_len][head_dim/2] (state.rope_cos/sin).
  * head_dim must be even and at most 512 (the reference's acc[512],
  * cpp/model.hpp:172) and n_heads a multiple of n_kv_heads (kv_mul,
- * cpp/model.hpp:295). 64 and 128 run on the MFMA kernels; other sizes on
- * plain VALU kernels with the same results contract (bit-exact K/V rows,
- * outputs within max-abs 2e-3 / rel 1e-2), where q, k and v need only 4-byte
- * and out 8-byte alignment. The cache starts zeroed, as the reference's
+ * cpp/model.hpp:295). 64 and 128 have MFMA kernels of their own; 80, 96,
+ * 112, 160, 192 and 256 run on general MFMA kernels (q and the attention
+ * weights as two fp16 parts, fp32 sums: fp32-level results) and every other
+ * size on plain VALU kernels, all with the same results contract (bit-exact
+ * K/V rows, outputs within max-abs 2e-3 / rel 1e-2). Sizes other than 64 and
+ * 128 need only 4-byte alignment of q, k and v and 8-byte of out. The cache starts zeroed, as the reference's
  * std::vector does. Besides the cache and the tables the context holds its
  * workspaces, the largest for the key ranges of a prompt: up to 256 rows of
  * head_dim + 2 floats per CU (34 MB at head size 128 on 256 CUs; 128 rows at the
@@ -104,9 +106,9 @@ int pqa_prefill(pqa_ctx* ctx, int layer, int start_pos, int n_tok, const float* 
  * pqa_decode that allocates nothing: the same kernels, with the split
  * partials in a static device array of the library (8 MiB per GPU, held until
  * the process ends; its address is taken once per device by pqa_create)
- * instead of the context's split workspace. Head sizes other than 64 and 128
- * also use the prepared-q buffer that pqa_create allocates (one token's q,
- * read and written, never grown by this call). No counterpart in the
+ * instead of the context's split workspace. The head sizes on the VALU kernels
+ * also use the prepared-q buffer that pqa_create allocates for them (one
+ * token's q, read and written, never grown by this call). No counterpart in the
  * reference: this entry point is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). Same arguments, results and errors as pqa_decode. The
@@ -355,13 +357,15 @@ int pqa_set_decode_split(pqa_ctx* ctx, int rows_per_split);
  * pqa_prefill_block) project K and V.
  * 1 (default): the attn_k and attn_v columns are computed in the reference's
  *    own summation order (vec_dot, cpp/quant.hpp:297-356, as forward_batch
- *    calls matmul_bias per token, cpp/model.hpp:503-546) on a VALU GEMM, so k
- *    and v are bit-identical to pqa_qkv_project's and the cache rows a prompt
+ *    calls matmul_bias per token, cpp/model.hpp:503-546), products and ordered
+ *    sums rounded one by one in fp32, so k and v are bit-identical to pqa_qkv_project's and the cache rows a prompt
  *    writes are the reference's bits (built without FMA contraction); q stays
  *    on the split fp16 GEMM, within its error bound (q only feeds scores).
- *    The first such call for a layer keeps its K/V rows as fp32, about
- *    2 * kv_dim * n_embd * 4 bytes (plus n_embd / 8 floats per row for Q8_0),
- *    until the weights are replaced.
+ *    The first such call for a layer keeps its K/V rows as fp32 (Q8_0: the
+ *    int8 values as floats, and the block scales) in the order the kernel
+ *    reads, about 2 * kv_dim * n_embd * 4 bytes (rows padded to tiles of 32,
+ *    columns to 64, for Q8_0 to 256; plus n_embd / 32 floats per row for
+ *    Q8_0), until the weights are replaced.
  * 0: all three on the split fp16 GEMM: faster, but a K or V element can land
  *    one fp16 step away from the reference's.
  * No counterpart in the reference, which has one order only.

@@ -17,12 +17,12 @@
 // 5 cycles but takes one of another wave in between (32 additions: 162 cycles
 // with one wave per SIMD, 80 per wave with two), so waves per SIMD count for
 // twice. The products come from v_mfma_f32_32x32x1_2b with C = 0, 2 x 32 x 32
-// of them round(w * x) in 70 cycles; it shares the vector ALU (no overlap was
+// of them round(w * x) in 65-72 cycles; it shares the vector ALU (no overlap was
 // measured), but takes its operands as one row and one token per lane where a
 // register tile reads 16 values for 64 products. Its bits are v_mul_f32's for
 // subnormals, infinities and NaN alike, up to the sign of a zero (2^27 products
-// of random and special bit patterns compared), which no sum that starts at +0
-// shows. (A shape with K > 1 would fuse its own additions and round otherwise.)
+// of random and special bit patterns compared; the tests send such inputs and weights
+// through the whole projection), which no sum that starts at +0 shows. (A shape with K > 1 would fuse its own additions and round otherwise.)
 //
 // ordered_kernel: a workgroup of 4 waves owns 32 tokens x 32 rows. The sums of a
 // (token, row) pair run as 8 independent sequences over 64-element stages:
@@ -40,7 +40,7 @@
 // Short prompts run 16 x 16 tiles with four sequences per wave (below).
 // K and V together, 2 x 1024 rows x 2560: 2048 tokens 353 us (a 64 x 64 register
 // tile with VALU multiplies, a launch each: 506 us), 75 tokens 26 us (226 us). 2048
-// tokens run at 163 cycles per MFMA and its 32 additions, against 141 measured for
+// tokens run at 163 cycles per MFMA and its 32 additions, against 143 measured for
 // the two alone at four waves per SIMD.
 //
 // Image of a matrix [rows][n] (n rounded up to whole stages, Q8_0 whole rounds,

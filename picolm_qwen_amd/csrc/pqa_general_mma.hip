@@ -13,25 +13,29 @@
 // operand of the second product. A last
 // half k-step of 16 dims (80, 112) takes v_mfma_f32_16x16x16_f16.
 //
-// K and V tiles of 64 keys (32 in a decode) arrive by direct global->LDS loads, 16-byte chunk c of
-// row r at slot c ^ x(r) (x within the largest power of two that divides the chunks
-// per row), free of bank conflicts for the K operand reads and the transposing V
-// reads alike.
+// K and V tiles of 64 keys (32 in a decode and at 256) arrive by direct global->LDS
+// loads, 16-byte chunk c of row r at slot c ^ x(r) (x within the largest power of two
+// that divides the chunks per row), free of bank conflicts for the K operand reads and
+// the transposing V reads alike.
 //   prefill  4 waves of 16 rows share each tile (two buffers, one barrier per
 //            tile);
 //   decode   the waves take a KV head's tiles in turn, each with two tiles of its
-//            own in flight behind the small operands; the wave with the last tile norms, rotates and rounds
-//            the new row, writes it to the cache and into its LDS tile. The waves'
-//            results meet in LDS.
+//            own in flight behind the small operands; the wave with the last tile
+//            norms, rotates and rounds the new row, writes it to the cache and into
+//            its LDS tile. The waves' results meet in LDS.
 // Either may cut the keys into ranges (workgroups) whose partials gen_merge_kernel
 // combines.
 //
-// Measured per layer against the VALU kernels (launch count, all kernels): decode of
-// 32 / 8 heads of 96 at 9000 44 -> 22 us (13 us for the 27.6 MB of cache, merge 4;
-// the rest is the gap between two launches), 8 / 2 heads of 256 at 4 37 -> 15 us;
+// Measured per layer against the VALU kernels, inputs changing from call to call:
+// decode of 32 / 8 heads of 96 at 9000 44 -> 22 us (13 us for the 27.6 MB of cache,
+// merge 4; the rest is the gap between two launches), 8 / 2 heads of 256 at 4 37 -> 16;
 // prefill of 700 tokens at head size 96 226 -> 41 us (kernel 207 -> 25; its bound is
-// the chain of one tile: operand reads, products, softmax, products), 851 tokens at
-// 256 353 -> 71. The error of a decode against 64-bit sums is 0.25 to 0.8 times theirs.
+// the chain of one tile: operand reads, products, softmax, products). The same inputs
+// again, 32 / 8 heads at 9000: 112 34.2 -> 17.7 us, 160 40.5 -> 21.8, 192 44.5 -> 23.6,
+// 256 53.4 -> 26.8 (at 32000 91.6 -> 57.2); one query head per KV head, 32 of 96 52.5 ->
+// 30.1, of 80 46.7 -> 29.1. The error against 64-bit sums over 75 decode and prefill
+// shapes is 0.45 to 1.01 times theirs. Other multiples of 16 up to 256 would fit the
+// template: each size is two kernels more, and no model that this library names has one.
 //
 // Infinities: a split product can turn inf into NaN (inf * 0, inf - inf), and a
 // masked key's V row still enters the product with weight 0. A row whose result is
@@ -105,12 +109,12 @@ __device__ __forceinline__ float4 gm_load4(const GenSrc& s, int t, int c, int ve
 
 // Four of a wave's rows again, rows row0 .. row0 + 3 of which those in `bad`: the rows
 // at q (fp32, prepared), each over its own keys of tiles first, first + step, ... below
-// end, in fp32. Row, m and l of each go to res, m_out and l_out in the
-// scale of the MFMA path (res may alias q). Lane = key for the scores (64 keys at a
-// time), lane = pair of dims for the sums over V, whose rows come 16 or 32 at a time,
-// ahead of the sums over those before; four rows share each K and V load. With an infinite V row in the cache (every row of a
-// wave again), per layer, the VALU kernels' time in brackets: 700 tokens of 32 / 8
-// heads of 96 270 us (210), 32 / 32 of 80 267 (340), 8 / 2 of 256 710 (272: 88
+// end, in fp32. Row, m and l of each go to res, m_out and l_out in the scale of the MFMA
+// path (res may alias q). Lane = key for the scores (64 keys at a time), lane = pair of
+// dims for the sums over V, whose rows come 16 or 32 at a time, ahead of the sums over
+// those before; four rows share each K and V load. With an infinite V row in the cache
+// (every row of a wave again), per layer, the VALU kernels' time in brackets: 700 tokens
+// of 32 / 8 heads of 96 270 us (210), 32 / 32 of 80 267 (340), 8 / 2 of 256 710 (272: 88
 // workgroups); decode at 9000 keys 21 (33), 55 (46) and 32 us (46). One row after the
 // other, each with K and V loads of its own, took 2460, 2390, 1900, 67, 157 and 38.
 template <int HD, int KEYS>
@@ -738,8 +742,14 @@ hipError_t launch_gen_mma(pqa_ctx* ctx, int layer, int start, int n_tok, const D
     a.ovec = ((uintptr_t)out & 15) == 0;
     a.qscale = 1.4426950408889634f / sqrtf((float)hd);
     // Ranges. Decode: about one workgroup per CU, each wave at least one 32-key tile; up
-    // to four tiles per wave need no second launch. Prefill: as long as the blocks
-    // leave CUs idle and a range keeps 512 keys (its q rows are prepared again).
+    // to four tiles per wave the second launch costs more than it gives (32 / 8 heads of
+    // 96: 384 keys 8.9 us in one launch and 10.0 in two, 512 9.9 and 10.1, 640 10.9 and
+    // 10.2; with the two waves of the sizes from 160 on the two meet at two tiles, 8 / 2
+    // heads of 256: 192 keys 15.7 and 14.8, 256 keys 17.6 and 14.9). Prefill: as long as
+    // the blocks leave CUs idle and a range keeps 512 keys, for each prepares its q rows
+    // again and is merged (32 / 8 heads of 96, ranges of 256, 512 and 1024 keys: 512 tokens
+    // at 0 29.9, 21.4 and 21.4 us, 64 tokens at 3000 28.2, 26.2 and 32.2; with two KV heads
+    // 256 is the better, 64 tokens at 2000 of 8 / 2 heads of 256 34.8, 45.3 and 67.0).
     const int tiles = (start + n_tok + 31) / 32;
     const long long wgs = (long long)a.nblk * a.n_kv;
     const int kw = decode ? (hd <= 128 ? 4 : 2) : 1;

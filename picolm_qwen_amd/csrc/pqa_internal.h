@@ -139,7 +139,7 @@ struct pqa_ctx {
 namespace pqa {
 
 // head sizes with MFMA kernels of their own; other even sizes up to 512 take the
-// general path, on the matrix cores for the sizes models use (pqa_general_mma.hip)
+// general path, six of them on the matrix cores (pqa_general_mma.hip)
 inline bool mfma_head_dim(int hd) { return hd == 64 || hd == 128; }
 inline bool gen_mma_head_dim(int hd) {
     return hd == 80 || hd == 96 || hd == 112 || hd == 160 || hd == 192 || hd == 256;

@@ -937,8 +937,10 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const float* __res
 // the chip; a prompt with fewer blocks finishes sooner with a block per
 // workgroup, and behind a long history with its keys in ranges. The estimate
 // counts steps of two key tiles (1.9 us): a block's prologue and epilogue take
-// about 3, and ranges a second launch that reads their partials; the partials
-// may take max_rows output rows. Measured per layer (32 / 8 heads of 128), pairs
+// about 3, and ranges a second launch that reads their partials, measured at 5 us or
+// 2.6 steps and charged as 6: the steps of the estimate are a few off, and three more
+// keep shapes out whose gain is within that. The partials may take max_rows output
+// rows. Measured per layer (32 / 8 heads of 128), pairs
 // against ranges: 300 tokens at 12000 400 -> 95 + 5 us (3 ranges, 240 workgroups
 // for 40), 1000 at 8000 322 -> 219, 40 at 30000 958 -> 68; 75 tokens at 0, one
 // block per workgroup, 21 -> 11.5; 2048 at 0 stay in pairs.

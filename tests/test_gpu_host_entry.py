@@ -76,7 +76,7 @@ def test_decode_host_successive_calls_and_a_failed_call():
     (16, 8, 128, 8191),    # whole-row workgroups, several splits: the merge launch writes out into host memory
     (16, 8, 128, 32767),   # Qwen3-1.7B shape at its full context
     (32, 4, 64, 2047),     # hd 64, several splits
-    (8, 2, 96, 3000),      # a general head size (VALU kernels, their own merge)
+    (8, 2, 96, 3000),      # a general head size (matrix-core kernel, its own merge)
 ])
 def test_decode_host_multi_split_and_general_equal_device_entry(nh, nkv, hd, pos):
     # the zero-copy host entry (kernels read q/k/v from and write out into the
