@@ -4,7 +4,9 @@ host cost of each launch.
 
 The calls to capture must allocate nothing and synchronise nothing:
 pqa_decode_noalloc is the entry point made for this (its split partials live
-in a static device array). A captured decode step is tied to its position
+in a static device array); pqa_prefill can be captured too (the buffer that a
+layer's first capture of few tokens behind a long history takes, it takes in the
+mode that allows it). A captured decode step is tied to its position
 (the launch shapes and arguments depend on it), so a caller keeps one graph
 per position, or re-captures. Replaying a step appends the same K/V row again
 (the same bits), so replays of one graph are idempotent.
