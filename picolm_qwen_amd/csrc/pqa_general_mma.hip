@@ -114,8 +114,8 @@ __device__ __forceinline__ float4 gm_load4(const GenSrc& s, int t, int c, int ve
 // dims for the sums over V, whose rows come 16 or 32 at a time, ahead of the sums over
 // those before; four rows share each K and V load. With an infinite V row in the cache
 // (every row of a wave again), per layer, the VALU kernels' time in brackets: 700 tokens
-// of 32 / 8 heads of 96 270 us (210), 32 / 32 of 80 267 (340), 8 / 2 of 256 710 (272: 88
-// workgroups); decode at 9000 keys 21 (33), 55 (46) and 32 us (46). One row after the
+// of 32 / 8 heads of 96 270 us (210), 32 / 32 of 80 267 (340), 8 / 2 of 256 439 (272: 88
+// workgroups); decode at 9000 keys 21 (33), 55 (46) and 27 us (46). One row after the
 // other, each with K and V loads of its own, took 2460, 2390, 1900, 67, 157 and 38.
 template <int HD, int KEYS>
 __device__ __forceinline__ void gen_rows(const GenMmaArgs& a, const uint16_t* kbase, const uint16_t* vbase, const float* q,
@@ -183,7 +183,7 @@ __device__ __forceinline__ void gen_rows(const GenMmaArgs& a, const uint16_t* kb
         const bool in = tile < end && key <= qlast;
         const u32x4* kr = (const u32x4*)(kbase + (size_t)(in ? key : kt * KEYS) * stride);
         float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 8
+#pragma unroll (NP == 1 ? 8 : 4)
         for (int c = 0; c < HD / 8; c++) {
             const u32x4 u = kr[c];
 #pragma unroll
